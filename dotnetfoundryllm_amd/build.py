@@ -42,7 +42,7 @@ def _run(cmd, cwd):
     return out
 
 
-DEVICE_SRCS = ["csrc/kernels.hip", "csrc/gemv.hip", "csrc/attention.hip", "csrc/prefill.hip", "csrc/api.hip"]
+DEVICE_SRCS = ["csrc/kernels.hip", "csrc/gemv.hip", "csrc/attention.hip", "csrc/prefill.hip", "csrc/pf_gemm8.hip", "csrc/api.hip"]
 
 
 def build_device_lib(verbose=False):

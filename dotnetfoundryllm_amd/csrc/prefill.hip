@@ -8,17 +8,12 @@
 // GEMM numerics: fp16 matrix cores (v_mfma_f32_16x16x32_f16, exact fp16 products summed in f32) on
 // operands of 22 significant bits. launch_pf_split scales each token row of X by a power of two so
 // that its largest magnitude lies in [2^14, 2^15) and writes hi = fp16(x) and lo = fp16(x - hi); the
-// epilogues undo the scale exactly. The weights enter in one of four forms:
-//  - Q4_K (pf_gemm_tile_q4k): sc q, an integer below 2048, exact in fp16; two products per weight,
-//    each 256-element block's sum scaled by its d in f32 and its min term one more product;
-//  - Q6_K (pf_gemm_tile_q6k): sc q as exact hi / lo fp16 integers; three products, d per block;
-//  - tile-interleaved Q8_0 (pf_gemm_tile_h): the int8 code q, exact in fp16; two products per
-//    weight, each 32-element block's sum scaled by its d in f32;
-//  - the other types (pf_gemm_tile_h): dequantized exactly (the Dequantizer arithmetic), scaled by
-//    a per-matrix power of two (pf_wexp) and split hi / lo; hi_x hi_w + hi_x lo_w + lo_x hi_w,
-//    within 2^-21 of the f32 product.
+// epilogues undo the scale exactly. Tile-interleaved weights enter as exact integers (pf_gemm8.hip); GGUF
+// rows (pf_gemm_tile_h) dequantized exactly (the Dequantizer arithmetic), scaled by a per-matrix power of
+// two (pf_wexp) and split hi / lo; hi_x hi_w + hi_x lo_w + lo_x hi_w, within 2^-21 of the f32 product.
 #include "prefill.hpp"
 #include "deq.hpp"
+#include "pf_gemm8.hpp"
 #include "gemv.hpp"
 
 #include <math.h>
@@ -61,156 +56,6 @@ __device__ __forceinline__ void pf_wave_sync() {
 // ---- exact dequantization of 32 weights [k0, k0 + 32) of row r (k0 a multiple of 32) -----------
 // load() fetches the raw bytes of the group (issued a K step ahead), deq() decodes them.
 template <int WT> struct PfW;
-
-// LAYOUT_TILES Q4_K (DequantizeQ4_K, Dequantizer.cs:251-294): group g of the row's block kb is the
-// 16 qs bytes of lane 16 (g & 3) + n in the region's first (g < 4) or second KiB; the row's header
-// (d, dmin, 12 scale bytes) sits at 2048 + 16 n.
-template <> struct PfW<FLLM_TYPE_Q4_K> {
-    struct Raw { uint4 qs, hdr; };
-    __device__ static void load(Raw& w4, const uint8_t* __restrict__ w, int K, int r, int k0) {
-        const int NB = K >> 8, kb = k0 >> 8, g = (k0 >> 5) & 7, n = r & 15;
-        const uint8_t* reg = w + ((size_t)(r >> 4) * NB + kb) * (16 * 144);
-        w4.qs = *(const uint4*)(reg + (g < 4 ? 0 : 1024) + 16 * (16 * (g & 3) + n));
-        w4.hdr = *(const uint4*)(reg + 2048 + 16 * n);
-    }
-    // byte idx of the 16-byte header
-    __device__ static uint32_t hbyte(const uint4& h, int idx) {
-        // selects of values, not of lvalues: a select of the fields' addresses keeps the header in
-        // scratch memory
-        const uint32_t x = h.x, y = h.y, z = h.z, w4 = h.w;
-        const uint32_t w = idx < 8 ? (idx < 4 ? x : y) : (idx < 12 ? z : w4);
-        return (w >> (8 * (idx & 3))) & 0xFFu;
-    }
-    // DecodeKScaleMin (Dequantizer.cs:506-521) on scale bytes 4..15 of the header
-    __device__ static void scale_min(const uint4& h, int g, int& sc, int& mn) {
-        if (g < 4) {
-            sc = (int)(hbyte(h, 4 + g) & 63u);
-            mn = (int)(hbyte(h, 8 + g) & 63u);
-        } else {
-            const uint32_t b = hbyte(h, 8 + g), lo = hbyte(h, g), hi = hbyte(h, 4 + g);
-            sc = (int)((b & 15u) | ((lo >> 6) << 4));
-            mn = (int)((b >> 4) | ((hi >> 6) << 4));
-        }
-    }
-    __device__ static void deq(const Raw& w4, const uint8_t*, int, int, int, int k0, float* v, float s = 1.0f) {
-        const int g = (k0 >> 5) & 7;
-        const float d = half_exact(w4.hdr.x & 0xFFFFu), dmin = half_exact(w4.hdr.x >> 16);
-        // DecodeKScaleMin (Dequantizer.cs:506-521) on scale bytes 4..15 of the header
-        int sc, mn;
-        if (g < 4) {
-            sc = (int)(hbyte(w4.hdr, 4 + g) & 63u);
-            mn = (int)(hbyte(w4.hdr, 8 + g) & 63u);
-        } else {
-            const uint32_t b = hbyte(w4.hdr, 8 + g), lo = hbyte(w4.hdr, g), hi = hbyte(w4.hdr, 4 + g);
-            sc = (int)((b & 15u) | ((lo >> 6) << 4));
-            mn = (int)((b >> 4) | ((hi >> 6) << 4));
-        }
-        // a power-of-two scale s commutes with the roundings: (dg s) q - mg s = s (dg q - mg) exactly
-        const float dg = d * (float)sc * s;
-        const float mg = dmin * (float)mn * s;
-        const uint32_t wd[4] = {w4.qs.x, w4.qs.y, w4.qs.z, w4.qs.w};
-#pragma unroll
-        for (int i = 0; i < 32; i++) {
-            const int at = q4t_pos(i >> 1);  // the tile layout's position of group byte i / 2
-            const uint32_t byte = (wd[at >> 2] >> (8 * (at & 3))) & 0xFFu;
-            const int q = (i & 1) ? (int)(byte >> 4) : (int)(byte & 15u);
-            v[i] = dg * (float)q - mg;
-        }
-    }
-};
-
-// LAYOUT_TILES Q6_K (DequantizeQ6_K, Dequantizer.cs:378-417): lane L = 16 (g & 3) + n holds ql of
-// group g (16 bytes, first or second KiB), qh of group g (8 bytes at 2048 + 16 L, +8 for g >= 4),
-// the group's two scales (bytes 0-1 or 2-3 of the dword at 3072 + 4 L); d at 3328 + 2 n.
-template <> struct PfW<FLLM_TYPE_Q6_K> {
-    struct Raw { uint4 ql; uint2 qh; uint32_t s4, d; };
-    __device__ static void load(Raw& w4, const uint8_t* __restrict__ w, int K, int r, int k0) {
-        const int NB = K >> 8, kb = k0 >> 8, g = (k0 >> 5) & 7, n = r & 15, L = 16 * (g & 3) + n;
-        const uint8_t* reg = w + ((size_t)(r >> 4) * NB + kb) * (16 * 210);
-        w4.ql = *(const uint4*)(reg + (g < 4 ? 0 : 1024) + 16 * L);
-        w4.qh = *(const uint2*)(reg + 2048 + 16 * L + (g < 4 ? 0 : 8));
-        w4.s4 = *(const uint32_t*)(reg + 3072 + 4 * L);
-        w4.d = *(const uint16_t*)(reg + 3328 + 2 * n);
-    }
-    __device__ static void deq(const Raw& w4, const uint8_t*, int, int, int, int k0, float* v, float s = 1.0f) {
-        const int g = (k0 >> 5) & 7;
-        const uint32_t sc2 = g < 4 ? (w4.s4 & 0xFFFFu) : (w4.s4 >> 16);
-        const float d = half_exact(w4.d) * s;
-        const uint32_t l4[4] = {w4.ql.x, w4.ql.y, w4.ql.z, w4.ql.w}, h2[2] = {w4.qh.x, w4.qh.y};
-#pragma unroll
-        for (int i = 0; i < 32; i++) {
-            const uint32_t lb = (l4[i >> 3] >> (8 * ((i >> 1) & 3))) & 0xFFu;
-            const int low = (i & 1) ? (int)(lb >> 4) : (int)(lb & 15u);
-            const uint32_t hb = (h2[i >> 4] >> (8 * ((i >> 2) & 3))) & 0xFFu;
-            const int high = (int)((hb >> (2 * (i & 3))) & 3u);
-            const int q = ((high << 4) | low) - 32;
-            const int scale = (int)(int8_t)((sc2 >> (8 * (i >> 4))) & 0xFFu);
-            v[i] = d * (float)scale * (float)q;
-        }
-    }
-};
-
-// LAYOUT_TILES Q8_0: block g & 3 (+4) of the row's chunk; its 32 int8 as two 16-byte pieces in
-// element order 4 by + j at byte 4 j + by; d of blocks q and q + 4 in one dword at 4096 + 16 n + 4 q
-template <> struct PfW<FLLM_TYPE_Q8_0> {
-    struct Raw { uint4 h0, h1; uint32_t d; };
-    __device__ static void load(Raw& w4, const uint8_t* __restrict__ w, int K, int r, int k0) {
-        const int NB = K >> 8, kb = k0 >> 8, g = (k0 >> 5) & 7, n = r & 15, q = g & 3, L = 16 * q + n;
-        const uint8_t* reg = w + ((size_t)(r >> 4) * NB + kb) * (16 * 272);
-        const uint8_t* base = reg + (g < 4 ? 0 : 2048) + 16 * L;
-        w4.h0 = *(const uint4*)base;
-        w4.h1 = *(const uint4*)(base + 1024);
-        w4.d = *(const uint32_t*)(reg + 4096 + 16 * n + 4 * q);
-    }
-    __device__ static void deq(const Raw& w4, const uint8_t*, int, int, int, int k0, float* v, float s = 1.0f) {
-        const int g = (k0 >> 5) & 7;
-        const float d = half_exact(g < 4 ? (w4.d & 0xFFFFu) : (w4.d >> 16)) * s;
-        const uint32_t hw[8] = {w4.h0.x, w4.h0.y, w4.h0.z, w4.h0.w, w4.h1.x, w4.h1.y, w4.h1.z, w4.h1.w};
-#pragma unroll
-        for (int e = 0; e < 32; e++) {
-            const int h = e >> 4, ee = e & 15, j = ee & 3, by = ee >> 2;  // byte 4 j + by of half h
-            v[e] = (float)(int8_t)((hw[4 * h + j] >> (8 * by)) & 0xFFu) * d;
-        }
-    }
-};
-
-// LAYOUT_TILES Q5_K: low nibbles as Q4_K, the group's regrouped high bits (bit 8 by + 4 h + j =
-// element 16 h + 4 by + j) in the dword at 2048 + 8 L (+4 for g >= 4), header at 2560 + 16 n
-template <> struct PfW<FLLM_TYPE_Q5_K> {
-    struct Raw { uint4 qs, hdr; uint32_t h; };
-    __device__ static void load(Raw& w4, const uint8_t* __restrict__ w, int K, int r, int k0) {
-        const int NB = K >> 8, kb = k0 >> 8, g = (k0 >> 5) & 7, n = r & 15, L = 16 * (g & 3) + n;
-        const uint8_t* reg = w + ((size_t)(r >> 4) * NB + kb) * (16 * 176);
-        w4.qs = *(const uint4*)(reg + (g < 4 ? 0 : 1024) + 16 * L);
-        w4.h = *(const uint32_t*)(reg + 2048 + 8 * L + (g < 4 ? 0 : 4));
-        w4.hdr = *(const uint4*)(reg + 2560 + 16 * n);
-    }
-    __device__ static void deq(const Raw& w4, const uint8_t*, int, int, int, int k0, float* v, float s = 1.0f) {
-        const int g = (k0 >> 5) & 7;
-        const float d = half_exact(w4.hdr.x & 0xFFFFu), dmin = half_exact(w4.hdr.x >> 16);
-        int sc, mn;
-        if (g < 4) {
-            sc = (int)(PfW<FLLM_TYPE_Q4_K>::hbyte(w4.hdr, 4 + g) & 63u);
-            mn = (int)(PfW<FLLM_TYPE_Q4_K>::hbyte(w4.hdr, 8 + g) & 63u);
-        } else {
-            const uint32_t b = PfW<FLLM_TYPE_Q4_K>::hbyte(w4.hdr, 8 + g), lo = PfW<FLLM_TYPE_Q4_K>::hbyte(w4.hdr, g),
-                           hi = PfW<FLLM_TYPE_Q4_K>::hbyte(w4.hdr, 4 + g);
-            sc = (int)((b & 15u) | ((lo >> 6) << 4));
-            mn = (int)((b >> 4) | ((hi >> 6) << 4));
-        }
-        // a power-of-two scale s commutes with the roundings: (dg s) q - mg s = s (dg q - mg) exactly
-        const float dg = d * (float)sc * s;
-        const float mg = dmin * (float)mn * s;
-        const uint32_t wd[4] = {w4.qs.x, w4.qs.y, w4.qs.z, w4.qs.w};
-#pragma unroll
-        for (int e = 0; e < 32; e++) {
-            const uint32_t byte = (wd[e >> 3] >> (8 * ((e >> 1) & 3))) & 0xFFu;
-            const int lo = (e & 1) ? (int)(byte >> 4) : (int)(byte & 15u);
-            const int hi = (int)((w4.h >> (8 * ((e >> 2) & 3) + 4 * (e >> 4) + (e & 3))) & 1u);
-            v[e] = dg * (float)((hi << 4) | lo) - mg;
-        }
-    }
-};
 
 // GGUF rows: elements e0 = r * K + k0 .. e0 + 31 of the flat block stream (K % 32 == 0, so the
 // group lies in one block of every format), decoded from memory when staged. PF_ROWS + type: one
@@ -406,7 +251,7 @@ __device__ __forceinline__ void pf_split8(const float* v, uint4& hi, uint4& lo) 
     lo = make_uint4(l[0], l[1], l[2], l[3]);
 }
 
-// Same tile as pf_gemm_tile: BM tokens x 128 weight rows, 4 waves of (BM / 2) x 64, K steps of 64.
+// Tile: BM tokens x 128 weight rows, 4 waves of (BM / 2) x 64, K steps of 64.
 // MFMA 16x16x32 f16: lane l supplies row (l & 15) of the A (tokens) and B (weight rows) tiles with
 // k = 8 (l >> 4) .. + 7 of a 32-wide slice, one 16-byte LDS read per operand and plane; D lane l holds
 // rows 4 (l >> 4) .. + 3 of column l & 15.
@@ -452,38 +297,7 @@ __device__ __forceinline__ void pf_gemm_tile_h(const PfGemm& a, const PfSeg& sg,
             const int c = tid + 256 * i, pl = c / (8 * BM), rem = c % (8 * BM);
             *(uint4*)(sx + ((size_t)pl * BM + (rem >> 3)) * PF_LDH + (rem & 7) * 8) = xr[i];
         }
-        if constexpr (WT == FLLM_TYPE_Q8_0) {
-            // exact-integer form: the int8 code q as an fp16 integer (its byte as 0x64 80 ^ byte =
-            // 1024 + 128 + q, minus 1152) in the weight plane, and the block's d' = d 2^-wexp (f32,
-            // exact) beside it; the products sum x hi q + x lo q per 32-element block and the block
-            // sum is added times d' in f32. Element 16 hh + 4 by + j is byte by of dword j of half hh,
-            // so a pair (e, e + 1) takes byte by of dwords j and j + 1.
-            const int k = k0 + 32 * wgrp;
-            uint32_t qv[16];
-            float dq = 0.0f;
-            if (wlive && k < a.K) {
-                const int g = (k >> 5) & 7;
-                dq = half_exact(g < 4 ? (wraw.d & 0xFFFFu) : (wraw.d >> 16)) * wsc;
-                const pf_hv2 off = {(_Float16)-1152.0f, (_Float16)-1152.0f};
-                const uint32_t wd[8] = {wraw.h0.x, wraw.h0.y, wraw.h0.z, wraw.h0.w, wraw.h1.x, wraw.h1.y, wraw.h1.z, wraw.h1.w};
-#pragma unroll
-                for (int pr = 0; pr < 16; pr++) {
-                    const int e = 2 * pr, hh = e >> 4, by = (e & 15) >> 2, j = e & 3;
-                    const uint32_t sel = 0x0C000C00u | ((uint32_t)(4 + by) << 16) | (uint32_t)by;
-                    const uint32_t p = __builtin_amdgcn_perm(wd[4 * hh + j + 1], wd[4 * hh + j], sel) ^ 0x64806480u;
-                    qv[pr] = __builtin_bit_cast(uint32_t, __builtin_bit_cast(pf_hv2, p) + off);
-                }
-            } else {
-#pragma unroll
-                for (int i = 0; i < 16; i++) qv[i] = 0u;
-            }
-            _Float16* d0 = sw + (size_t)wrow * PF_LDH + 32 * wgrp;
-#pragma unroll
-            for (int i = 0; i < 4; i++)
-                *(uint4*)(d0 + 8 * i) = make_uint4(qv[4 * i], qv[4 * i + 1], qv[4 * i + 2], qv[4 * i + 3]);
-            // the block scales in the second weight plane, which this form leaves free
-            ((float*)(sw + (size_t)PF_BN * PF_LDH))[wgrp * PF_BN + wrow] = dq;
-        } else {
+        {
             float v[32];
             const int k = k0 + 32 * wgrp;
             if (wlive && k < a.K) {
@@ -505,44 +319,6 @@ __device__ __forceinline__ void pf_gemm_tile_h(const PfGemm& a, const PfSeg& sg,
         // the next step's global loads fly while this step multiplies
         if (k0 + PF_BK < ke) fetch(k0 + PF_BK);
         __syncthreads();
-        if constexpr (WT == FLLM_TYPE_Q8_0) {
-            const float* sdq = (const float*)(sw + (size_t)PF_BN * PF_LDH);
-#pragma unroll
-            for (int kk = 0; kk < PF_BK; kk += 32) {
-                const int ko = kk + 8 * (lane >> 4);
-                pf_h8 ah[TI], al[TI], bq[4];
-                float dj[4];
-#pragma unroll
-                for (int i = 0; i < TI; i++) {
-                    const _Float16* p = sx + (size_t)(WM * wm + 16 * i + (lane & 15)) * PF_LDH + ko;
-                    ah[i] = *(const pf_h8*)p;
-                    al[i] = *(const pf_h8*)(p + (size_t)BM * PF_LDH);
-                }
-#pragma unroll
-                for (int j = 0; j < 4; j++) {
-                    const int r = 64 * wn + 16 * j + (lane & 15);
-                    bq[j] = *(const pf_h8*)(sw + (size_t)r * PF_LDH + ko);
-                    dj[j] = sdq[(kk >> 5) * PF_BN + r];
-                }
-                // the block's sum (x lo q, then x hi q) over all tiles in turn, then its d' times it
-                pf_f32x4 bs[TI][4];
-#pragma unroll
-                for (int i = 0; i < TI; i++)
-#pragma unroll
-                    for (int j = 0; j < 4; j++)
-                        bs[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(al[i], bq[j], pf_f32x4{0.0f, 0.0f, 0.0f, 0.0f}, 0, 0, 0);
-#pragma unroll
-                for (int i = 0; i < TI; i++)
-#pragma unroll
-                    for (int j = 0; j < 4; j++) bs[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ah[i], bq[j], bs[i][j], 0, 0, 0);
-#pragma unroll
-                for (int i = 0; i < TI; i++)
-#pragma unroll
-                    for (int j = 0; j < 4; j++)
-#pragma unroll
-                        for (int e = 0; e < 4; e++) acc[i][j][e] = fmaf(dj[j], bs[i][j][e], acc[i][j][e]);
-            }
-        } else {
 #pragma unroll
         for (int kk = 0; kk < PF_BK; kk += 32) {
             const int ko = kk + 8 * (lane >> 4);
@@ -574,7 +350,6 @@ __device__ __forceinline__ void pf_gemm_tile_h(const PfGemm& a, const PfSeg& sg,
 #pragma unroll
                 for (int j = 0; j < 4; j++) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ah[i], bh[j], acc[i][j], 0, 0, 0);
         }
-        }
     }
     const float wun = ldexpf(1.0f, sg.wexp);
 #pragma unroll
@@ -598,526 +373,6 @@ __device__ __forceinline__ void pf_gemm_tile_h(const PfGemm& a, const PfSeg& sg,
                 }
             }
         }
-}
-
-// ---- fp16 form, Q4_K -------------------------------------------------------------------------
-// A Q4_K weight is dg q - mg with dg = d sc_g, mg = dmin m_g (Dequantizer.cs:251-294), so
-//   sum_i w_i x_i = d sum_(g in block) sum_(i in g) (sc_g q_i) x_i - sum_g (dmin m_g) X_g,
-// X_g the sum of group g's x. sc_g q_i <= 945 is an integer, exact in fp16: the weights need no split
-// and a product is two MFMAs (x hi and x lo against the same weights). Every 256-element block's sum
-// is scaled by its d in f32; the min term of a block is one more MFMA whose K slice packs, per row,
-// (v_g hi, v_g lo, v_g hi) for v_g = -dmin m_g against, per token, (X_g hi, X_g hi, X_g lo), the
-// three products of the two splits, added to the same accumulator. The group sums are stored times
-// 2^-6 (to stay in fp16's range) and v_g taken times 2^6, so their products are unchanged.
-// LDS row stride (halves) of a block's min-term slice: its three used 16-byte chunks (the fourth
-// of the MFMA's K slice is zero and is not stored: the lanes that would read it take zeros)
-constexpr int PF_LDV = 24;
-
-template <int BM>
-static constexpr size_t pf_gemm_lds_k() {
-    return sizeof(_Float16) * ((size_t)(2 * BM + PF_BN) * PF_LDH + (size_t)(BM + PF_BN) * PF_LDV) + sizeof(float) * PF_BN;
-}
-
-// sc q_i for the 8 elements of one qs dword (bytes b = 0..3: element 2 b the low nibble, 2 b + 1 the
-// high one), as 4 dwords of fp16 pairs: 1024 + q by setting the fp16 pattern 0x6400 | q, minus 1024,
-// times sc, all exact
-__device__ __forceinline__ void pf_q4_pairs(uint32_t x, pf_hv2 sc2, uint32_t* out) {
-    const uint32_t lo = x & 0x0F0F0F0Fu, hi = (x >> 4) & 0x0F0F0F0Fu;
-    // (1024 + q) sc - 1024 sc in one fma: exact, the result sc q being an integer below 2048
-    const pf_hv2 nb = sc2 * pf_hv2{(_Float16)-1024.0f, (_Float16)-1024.0f};
-#pragma unroll
-    for (int b = 0; b < 4; b++) {
-        // bytes: low nibble of byte b, 0, high nibble of byte b, 0
-        const uint32_t sel = 0x0C000C00u | ((uint32_t)(4 + b) << 16) | (uint32_t)b;
-        const uint32_t p = __builtin_amdgcn_perm(hi, lo, sel) | 0x64006400u;
-        const pf_hv2 v = __builtin_elementwise_fma(__builtin_bit_cast(pf_hv2, p), sc2, nb);
-        out[b] = __builtin_bit_cast(uint32_t, v);
-    }
-}
-
-// Q5_K: the same for 5-bit codes (sc q <= 63 * 31 < 2048, still exact). The group's regrouped
-// high-bit dword h holds element 16 hf + 4 by + j at bit 8 by + 4 hf + j: the pair (2 b, 2 b + 1)
-// of qs dword u has its high bits at bits p, p + 1 of the half (u & 1) of h, p = 8 (b >> 1) +
-// 4 (u >> 1) + 2 (b & 1) < 15. With z = h16 | h16 << 15 for that 16-bit half, (z >> p) puts them at
-// bits 0 and 16.
-template <int U>
-__device__ __forceinline__ void pf_q5_pairs(uint32_t x, uint32_t z, pf_hv2 sc2, uint32_t* out) {
-    const uint32_t lo = x & 0x0F0F0F0Fu, hi = (x >> 4) & 0x0F0F0F0Fu;
-    const pf_hv2 nb = sc2 * pf_hv2{(_Float16)-1024.0f, (_Float16)-1024.0f};
-#pragma unroll
-    for (int b = 0; b < 4; b++) {
-        const uint32_t sel = 0x0C000C00u | ((uint32_t)(4 + b) << 16) | (uint32_t)b;
-        const int pos = 8 * (b >> 1) + 4 * (U >> 1) + 2 * (b & 1);
-        const uint32_t t = (pos >= 4 ? (z >> (pos - 4)) : (z << (4 - pos))) & 0x00100010u;
-        const uint32_t p = __builtin_amdgcn_perm(hi, lo, sel) | t | 0x64006400u;
-        const pf_hv2 v = __builtin_elementwise_fma(__builtin_bit_cast(pf_hv2, p), sc2, nb);
-        out[b] = __builtin_bit_cast(uint32_t, v);
-    }
-}
-
-// WT: FLLM_TYPE_Q4_K or FLLM_TYPE_Q5_K (same header, scales and block structure)
-template <int BM, int WT = FLLM_TYPE_Q4_K>
-__device__ __forceinline__ void pf_gemm_tile_q4k(const PfGemm& a, const PfSeg& sg, int n0, int t0, _Float16* lds) {
-    constexpr int WM = BM / 2, TI = WM / 16;
-    _Float16* sx = lds;                                    // [2][BM][PF_LDH]
-    _Float16* sw = sx + (size_t)2 * BM * PF_LDH;           // [PF_BN][PF_LDH]
-    _Float16* sav = sw + (size_t)PF_BN * PF_LDH;           // [BM][PF_LDV]
-    _Float16* swv = sav + (size_t)BM * PF_LDV;             // [PF_BN][PF_LDV]
-    float* sd = (float*)(swv + (size_t)PF_BN * PF_LDV);    // [PF_BN]
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int wm = wave >> 1, wn = wave & 1;
-    pf_f32x4 acc[TI][4], blk[TI][4];
-#pragma unroll
-    for (int i = 0; i < TI; i++)
-#pragma unroll
-        for (int j = 0; j < 4; j++) acc[i][j] = blk[i][j] = pf_f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-
-    constexpr int XP = BM * 16 / 256;
-    const size_t plane = (size_t)a.T * a.ldh;
-    const int G = a.K / 32;
-    const _Float16* xg = a.xh + 2 * plane;  // group sums: hi plane, then lo plane
-    const size_t gplane = (size_t)a.T * G;
-    const int wrow = tid & (PF_BN - 1), wgrp = tid / PF_BN, wr = n0 + wrow;
-    const bool wlive = wr < sg.N;
-    // block-start extras: token row (tid >> 1) of the min-term slice, its hi (tid even) or lo group sums
-    const int vt = tid >> 1, vhl = tid & 1;
-    using Raw = typename PfW<WT>::Raw;
-    uint4 xr[XP], xv = make_uint4(0u, 0u, 0u, 0u);
-    Raw wraw;
-    // a tile of BM whole token rows (uniform over the workgroup) loads without the row test
-    const bool full = t0 + BM <= a.T;
-    auto fetch = [&](int k0) {
-        if (full) {
-#pragma unroll
-            for (int i = 0; i < XP; i++) {
-                const int c = tid + 256 * i, pl = c / (8 * BM), rem = c % (8 * BM);
-                xr[i] = *(const uint4*)(a.xh + pl * plane + (size_t)(t0 + (rem >> 3)) * a.ldh + k0 + (rem & 7) * 8);
-            }
-        } else {
-#pragma unroll
-            for (int i = 0; i < XP; i++) {
-                const int c = tid + 256 * i, pl = c / (8 * BM), rem = c % (8 * BM), t = t0 + (rem >> 3);
-                xr[i] = t < a.T ? *(const uint4*)(a.xh + pl * plane + (size_t)t * a.ldh + k0 + (rem & 7) * 8)
-                                : make_uint4(0u, 0u, 0u, 0u);
-            }
-        }
-        if ((k0 & 255) == 0 && vt < BM) {
-            const int t = t0 + vt;
-            xv = t < a.T ? *(const uint4*)(xg + vhl * gplane + (size_t)t * G + (k0 >> 5)) : make_uint4(0u, 0u, 0u, 0u);
-        }
-        if (wlive) PfW<WT>::load(wraw, sg.w, a.K, wr, k0 + 32 * wgrp);
-    };
-    // whole 256-element blocks (K and the split parts are multiples of 256): four K steps per block,
-    // the block's end straight-line after them, so the accumulators stay in place across steps
-    const int kb = (int)blockIdx.z * a.kpart, ke = kb + a.kpart < a.K ? kb + a.kpart : a.K;
-    fetch(kb);
-    for (int kblk = kb; kblk < ke; kblk += 256) {
-#pragma unroll
-        for (int st = 0; st < 4; st++) {
-            const int k0 = kblk + st * PF_BK;
-            __syncthreads();  // the previous step's operands have been read
-#pragma unroll
-            for (int i = 0; i < XP; i++) {
-                const int c = tid + 256 * i, pl = c / (8 * BM), rem = c % (8 * BM);
-                *(uint4*)(sx + ((size_t)pl * BM + (rem >> 3)) * PF_LDH + (rem & 7) * 8) = xr[i];
-            }
-            const int g = 2 * st + wgrp;
-            {
-                uint32_t out[16];
-                if (wlive) {
-                    int sc, mn;
-                    PfW<FLLM_TYPE_Q4_K>::scale_min(wraw.hdr, g, sc, mn);
-                    const _Float16 sch = (_Float16)(float)sc;
-                    const pf_hv2 sc2 = {sch, sch};
-                    if constexpr (WT == FLLM_TYPE_Q5_K) {
-                        const uint32_t h0 = wraw.h & 0xFFFFu, h1 = wraw.h >> 16;
-                        const uint32_t z0 = h0 | (h0 << 15), z1 = h1 | (h1 << 15);
-                        pf_q5_pairs<0>(wraw.qs.x, z0, sc2, out);
-                        pf_q5_pairs<1>(wraw.qs.y, z1, sc2, out + 4);
-                        pf_q5_pairs<2>(wraw.qs.z, z0, sc2, out + 8);
-                        pf_q5_pairs<3>(wraw.qs.w, z1, sc2, out + 12);
-                    } else {
-                        // the tile layout's dwords of a half: its bytes 0, 2, 4, 6 and 1, 3, 5, 7
-                        // (element pairs 0, 2, 4, 6 and 1, 3, 5, 7 of the half)
-                        uint32_t ev[4], od[4];
-#pragma unroll
-                        for (int hf = 0; hf < 2; hf++) {
-                            pf_q4_pairs(hf ? wraw.qs.z : wraw.qs.x, sc2, ev);
-                            pf_q4_pairs(hf ? wraw.qs.w : wraw.qs.y, sc2, od);
-#pragma unroll
-                            for (int b = 0; b < 4; b++) {
-                                out[8 * hf + 2 * b] = ev[b];
-                                out[8 * hf + 2 * b + 1] = od[b];
-                            }
-                        }
-                    }
-                } else {
-#pragma unroll
-                    for (int i = 0; i < 16; i++) out[i] = 0u;
-                }
-                uint4* dst = (uint4*)(sw + (size_t)wrow * PF_LDH + 32 * wgrp);
-#pragma unroll
-                for (int i = 0; i < 4; i++) dst[i] = make_uint4(out[4 * i], out[4 * i + 1], out[4 * i + 2], out[4 * i + 3]);
-            }
-            if (st == 0) {
-                // the block's d and min-term slice of this row (v_g = -dmin m_g, exact in f32, split)
-                if (wgrp == 0) {
-                    const float d = wlive ? half_exact(wraw.hdr.x & 0xFFFFu) : 0.0f;
-                    const float dmin = wlive ? half_exact(wraw.hdr.x >> 16) : 0.0f;
-                    sd[wrow] = d;
-                    uint32_t vh[4], vl[4];
-#pragma unroll
-                    for (int gg = 0; gg < 8; gg += 2) {
-                        int sc0, mn0, sc1, mn1;
-                        PfW<FLLM_TYPE_Q4_K>::scale_min(wraw.hdr, gg, sc0, mn0);
-                        PfW<FLLM_TYPE_Q4_K>::scale_min(wraw.hdr, gg + 1, sc1, mn1);
-                        const float v0 = wlive ? -(dmin * (float)mn0) * 64.0f : 0.0f;
-                        const float v1 = wlive ? -(dmin * (float)mn1) * 64.0f : 0.0f;
-                        const pf_h2 h = __builtin_amdgcn_cvt_pkrtz(v0, v1);
-                        const pf_h2 l = __builtin_amdgcn_cvt_pkrtz(v0 - (float)h[0], v1 - (float)h[1]);
-                        vh[gg >> 1] = __builtin_bit_cast(uint32_t, h);
-                        vl[gg >> 1] = __builtin_bit_cast(uint32_t, l);
-                    }
-                    uint4* dv = (uint4*)(swv + (size_t)wrow * PF_LDV);
-                    dv[0] = make_uint4(vh[0], vh[1], vh[2], vh[3]);
-                    dv[1] = make_uint4(vl[0], vl[1], vl[2], vl[3]);
-                    dv[2] = dv[0];
-                }
-                // tokens: (X hi, X hi, X lo, 0) against (v hi, v lo, v hi, 0)
-                if (vt < BM) {
-                    uint4* av = (uint4*)(sav + (size_t)vt * PF_LDV);
-                    if (vhl == 0) {
-                        av[0] = xv;
-                        av[1] = xv;
-                    } else {
-                        av[2] = xv;
-                    }
-                }
-            }
-            if (k0 + PF_BK < ke) fetch(k0 + PF_BK);
-            __syncthreads();
-#pragma unroll
-            for (int kk = 0; kk < PF_BK; kk += 32) {
-                const int ko = kk + 8 * (lane >> 4);
-                pf_h8 ah[TI], al[TI], bw[4];
-#pragma unroll
-                for (int i = 0; i < TI; i++) {
-                    const _Float16* p = sx + (size_t)(WM * wm + 16 * i + (lane & 15)) * PF_LDH + ko;
-                    ah[i] = *(const pf_h8*)p;
-                    al[i] = *(const pf_h8*)(p + (size_t)BM * PF_LDH);
-                }
-#pragma unroll
-                for (int j = 0; j < 4; j++) bw[j] = *(const pf_h8*)(sw + (size_t)(64 * wn + 16 * j + (lane & 15)) * PF_LDH + ko);
-                // the block's first product starts its sum from zero
-#pragma unroll
-                for (int i = 0; i < TI; i++)
-#pragma unroll
-                    for (int j = 0; j < 4; j++)
-                        blk[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(
-                            al[i], bw[j], (st == 0 && kk == 0) ? pf_f32x4{0.0f, 0.0f, 0.0f, 0.0f} : blk[i][j], 0, 0, 0);
-#pragma unroll
-                for (int i = 0; i < TI; i++)
-#pragma unroll
-                    for (int j = 0; j < 4; j++) blk[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ah[i], bw[j], blk[i][j], 0, 0, 0);
-            }
-        }
-        // the block's d times its sum, and its min term (sd / sav / swv were written at the block's
-        // first step and are rewritten only after the next block's first barrier)
-        const int ko = 8 * (lane >> 4);
-        const bool kz = (lane >> 4) == 3;  // the slice's fourth chunk: zeros
-        const pf_h8 z8 = {};
-        pf_h8 av[TI], bv[4];
-#pragma unroll
-        for (int i = 0; i < TI; i++)
-            av[i] = kz ? z8 : *(const pf_h8*)(sav + (size_t)(WM * wm + 16 * i + (lane & 15)) * PF_LDV + (kz ? 0 : ko));
-#pragma unroll
-        for (int j = 0; j < 4; j++)
-            bv[j] = kz ? z8 : *(const pf_h8*)(swv + (size_t)(64 * wn + 16 * j + (lane & 15)) * PF_LDV + (kz ? 0 : ko));
-#pragma unroll
-        for (int j = 0; j < 4; j++) {
-            const float d = sd[64 * wn + 16 * j + (lane & 15)];
-#pragma unroll
-            for (int i = 0; i < TI; i++) {
-#pragma unroll
-                for (int e = 0; e < 4; e++) acc[i][j][e] = fmaf(d, blk[i][j][e], acc[i][j][e]);
-                acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(av[i], bv[j], acc[i][j], 0, 0, 0);
-            }
-        }
-    }
-#pragma unroll
-    for (int i = 0; i < TI; i++)
-#pragma unroll
-        for (int e = 0; e < 4; e++) {
-            const int t = t0 + WM * wm + 16 * i + 4 * (lane >> 4) + e;
-            if (t >= a.T) continue;
-            const float f = a.xs[t];  // undoes the activations' scale: exact
-#pragma unroll
-            for (int j = 0; j < 4; j++) {
-                const int n = n0 + 64 * wn + 16 * j + (lane & 15);
-                if (n >= sg.N) continue;
-                const float r = acc[i][j][e] * f;
-                if (blockIdx.z == 0) {
-                    float* p = sg.y + (size_t)t * sg.ldy + n;
-                    *p = a.add ? *p + r : r;
-                } else {
-                    const size_t col = (size_t)(sg.y - a.seg[0].y);
-                    a.part[(size_t)(blockIdx.z - 1) * a.T * sg.ldy + (size_t)t * sg.ldy + col + n] = r;
-                }
-            }
-        }
-}
-
-// ---- fp16 form, Q6_K --------------------------------------------------------------------------
-// A Q6_K weight is d (sc q) with q = v - 32 (v the 6-bit code) and sc the int8 scale of its 16
-// elements (Dequantizer.cs:378-417). I = sc q is an integer of magnitude at most 4096: hi = fp16(I)
-// (exact up to 2048, even integers above) and lo = I - hi (0 or +-1) hold it exactly. A block's sum
-// is x hi * I hi + x lo * I hi + x hi * I lo (the dropped x lo * I lo is below 2^-22 of a product),
-// accumulated apart and added times the block's d in f32 at its end. The weights need no matrix
-// scale: the epilogue only undoes the activations' power of two.
-template <int BM>
-static constexpr size_t pf_gemm_lds_q6() {
-    return sizeof(_Float16) * (size_t)(2 * BM + 2 * PF_BN) * PF_LDH + sizeof(float) * PF_BN;
-}
-
-// the 8 elements of ql dword x (element 2 b: low nibble of byte b, 2 b + 1: high nibble) with their
-// high bits (element j: bits 2 j, 2 j + 1 of h16), scale pair sc2: hi and lo halves of sc q as 4
-// fp16 pairs each. A pair's code v goes into fp16 1024 + v (nibble at bits 0-3, high bits at 4-5 of
-// each half, pattern 0x6400), minus 1056 gives q exactly.
-__device__ __forceinline__ void pf_q6_pairs(uint32_t x, uint32_t h16, pf_hv2 sc2, uint32_t* hi, uint32_t* lo) {
-    const uint32_t nl = x & 0x0F0F0F0Fu, nh = (x >> 4) & 0x0F0F0F0Fu;
-    // y >> 4 b: bits 0-1 the high bits of element 2 b, bits 16-17 those of element 2 b + 1
-    const uint32_t y = h16 | (h16 << 14);
-    const pf_hv2 off = {(_Float16)-1056.0f, (_Float16)-1056.0f};
-#pragma unroll
-    for (int b = 0; b < 4; b++) {
-        const uint32_t sel = 0x0C000C00u | ((uint32_t)(4 + b) << 16) | (uint32_t)b;
-        const uint32_t t = (b == 0 ? (y << 4) : (y >> (4 * b - 4))) & 0x00300030u;
-        const uint32_t p = __builtin_amdgcn_perm(nh, nl, sel) | t | 0x64006400u;
-        const pf_hv2 q = __builtin_bit_cast(pf_hv2, p) + off;
-        const pf_hv2 vh = q * sc2;
-        const pf_hv2 vl = __builtin_elementwise_fma(q, sc2, -vh);
-        hi[b] = __builtin_bit_cast(uint32_t, vh);
-        lo[b] = __builtin_bit_cast(uint32_t, vl);
-    }
-}
-
-// Same tile and step structure as pf_gemm_tile_q4k (whole 256-element blocks, four K steps each);
-// the weights go into LDS as hi / lo planes.
-template <int BM>
-__device__ __forceinline__ void pf_gemm_tile_q6k(const PfGemm& a, const PfSeg& sg, int n0, int t0, _Float16* lds) {
-    constexpr int WM = BM / 2, TI = WM / 16;
-    _Float16* sx = lds;                                    // [2][BM][PF_LDH]
-    _Float16* sw = sx + (size_t)2 * BM * PF_LDH;           // [2][PF_BN][PF_LDH]
-    float* sd = (float*)(sw + (size_t)2 * PF_BN * PF_LDH);  // [PF_BN]
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int wm = wave >> 1, wn = wave & 1;
-    pf_f32x4 acc[TI][4], blk[TI][4];
-#pragma unroll
-    for (int i = 0; i < TI; i++)
-#pragma unroll
-        for (int j = 0; j < 4; j++) acc[i][j] = blk[i][j] = pf_f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-
-    constexpr int XP = BM * 16 / 256;
-    const size_t plane = (size_t)a.T * a.ldh;
-    const int wrow = tid & (PF_BN - 1), wgrp = tid / PF_BN, wr = n0 + wrow;
-    const bool wlive = wr < sg.N;
-    using Raw = typename PfW<FLLM_TYPE_Q6_K>::Raw;
-    uint4 xr[XP];
-    Raw wraw;
-    const bool full = t0 + BM <= a.T;
-    auto fetch = [&](int k0) {
-        if (full) {
-#pragma unroll
-            for (int i = 0; i < XP; i++) {
-                const int c = tid + 256 * i, pl = c / (8 * BM), rem = c % (8 * BM);
-                xr[i] = *(const uint4*)(a.xh + pl * plane + (size_t)(t0 + (rem >> 3)) * a.ldh + k0 + (rem & 7) * 8);
-            }
-        } else {
-#pragma unroll
-            for (int i = 0; i < XP; i++) {
-                const int c = tid + 256 * i, pl = c / (8 * BM), rem = c % (8 * BM), t = t0 + (rem >> 3);
-                xr[i] = t < a.T ? *(const uint4*)(a.xh + pl * plane + (size_t)t * a.ldh + k0 + (rem & 7) * 8)
-                                : make_uint4(0u, 0u, 0u, 0u);
-            }
-        }
-        if (wlive) PfW<FLLM_TYPE_Q6_K>::load(wraw, sg.w, a.K, wr, k0 + 32 * wgrp);
-    };
-    const int kb = (int)blockIdx.z * a.kpart, ke = kb + a.kpart < a.K ? kb + a.kpart : a.K;
-    fetch(kb);
-    for (int kblk = kb; kblk < ke; kblk += 256) {
-#pragma unroll
-        for (int st = 0; st < 4; st++) {
-            const int k0 = kblk + st * PF_BK;
-            __syncthreads();  // the previous step's operands have been read
-#pragma unroll
-            for (int i = 0; i < XP; i++) {
-                const int c = tid + 256 * i, pl = c / (8 * BM), rem = c % (8 * BM);
-                *(uint4*)(sx + ((size_t)pl * BM + (rem >> 3)) * PF_LDH + (rem & 7) * 8) = xr[i];
-            }
-            const int g = 2 * st + wgrp;
-            {
-                uint32_t hv[16], lv[16];
-                if (wlive) {
-                    const uint32_t sc = g < 4 ? (wraw.s4 & 0xFFFFu) : (wraw.s4 >> 16);
-                    const pf_hv2 sa = {(_Float16)(float)(int)(int8_t)(sc & 0xFFu), (_Float16)(float)(int)(int8_t)(sc & 0xFFu)};
-                    const pf_hv2 sb = {(_Float16)(float)(int)(int8_t)(sc >> 8), (_Float16)(float)(int)(int8_t)(sc >> 8)};
-                    pf_q6_pairs(wraw.ql.x, wraw.qh.x & 0xFFFFu, sa, hv, lv);
-                    pf_q6_pairs(wraw.ql.y, wraw.qh.x >> 16, sa, hv + 4, lv + 4);
-                    pf_q6_pairs(wraw.ql.z, wraw.qh.y & 0xFFFFu, sb, hv + 8, lv + 8);
-                    pf_q6_pairs(wraw.ql.w, wraw.qh.y >> 16, sb, hv + 12, lv + 12);
-                } else {
-#pragma unroll
-                    for (int i = 0; i < 16; i++) hv[i] = lv[i] = 0u;
-                }
-                uint4* dh = (uint4*)(sw + (size_t)wrow * PF_LDH + 32 * wgrp);
-                uint4* dl = (uint4*)(sw + (size_t)(PF_BN + wrow) * PF_LDH + 32 * wgrp);
-#pragma unroll
-                for (int i = 0; i < 4; i++) {
-                    dh[i] = make_uint4(hv[4 * i], hv[4 * i + 1], hv[4 * i + 2], hv[4 * i + 3]);
-                    dl[i] = make_uint4(lv[4 * i], lv[4 * i + 1], lv[4 * i + 2], lv[4 * i + 3]);
-                }
-            }
-            if (st == 0 && wgrp == 0) sd[wrow] = wlive ? half_exact(wraw.d & 0xFFFFu) : 0.0f;
-            if (k0 + PF_BK < ke) fetch(k0 + PF_BK);
-            __syncthreads();
-#pragma unroll
-            for (int kk = 0; kk < PF_BK; kk += 32) {
-                const int ko = kk + 8 * (lane >> 4);
-                pf_h8 ah[TI], al[TI], bh[4], bl[4];
-#pragma unroll
-                for (int i = 0; i < TI; i++) {
-                    const _Float16* p = sx + (size_t)(WM * wm + 16 * i + (lane & 15)) * PF_LDH + ko;
-                    ah[i] = *(const pf_h8*)p;
-                    al[i] = *(const pf_h8*)(p + (size_t)BM * PF_LDH);
-                }
-#pragma unroll
-                for (int j = 0; j < 4; j++) {
-                    const _Float16* p = sw + (size_t)(64 * wn + 16 * j + (lane & 15)) * PF_LDH + ko;
-                    bh[j] = *(const pf_h8*)p;
-                    bl[j] = *(const pf_h8*)(p + (size_t)PF_BN * PF_LDH);
-                }
-                // the block's first product starts its sum from zero
-#pragma unroll
-                for (int i = 0; i < TI; i++)
-#pragma unroll
-                    for (int j = 0; j < 4; j++)
-                        blk[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(
-                            al[i], bh[j], (st == 0 && kk == 0) ? pf_f32x4{0.0f, 0.0f, 0.0f, 0.0f} : blk[i][j], 0, 0, 0);
-#pragma unroll
-                for (int i = 0; i < TI; i++)
-#pragma unroll
-                    for (int j = 0; j < 4; j++) blk[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ah[i], bl[j], blk[i][j], 0, 0, 0);
-#pragma unroll
-                for (int i = 0; i < TI; i++)
-#pragma unroll
-                    for (int j = 0; j < 4; j++) blk[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ah[i], bh[j], blk[i][j], 0, 0, 0);
-            }
-        }
-        // the block's d times its sum (sd was written at the block's first step and is rewritten only
-        // after the next block's first barrier)
-#pragma unroll
-        for (int j = 0; j < 4; j++) {
-            const float d = sd[64 * wn + 16 * j + (lane & 15)];
-#pragma unroll
-            for (int i = 0; i < TI; i++)
-#pragma unroll
-                for (int e = 0; e < 4; e++) acc[i][j][e] = fmaf(d, blk[i][j][e], acc[i][j][e]);
-        }
-    }
-#pragma unroll
-    for (int i = 0; i < TI; i++)
-#pragma unroll
-        for (int e = 0; e < 4; e++) {
-            const int t = t0 + WM * wm + 16 * i + 4 * (lane >> 4) + e;
-            if (t >= a.T) continue;
-            const float f = a.xs[t];  // undoes the activations' scale: exact
-#pragma unroll
-            for (int j = 0; j < 4; j++) {
-                const int n = n0 + 64 * wn + 16 * j + (lane & 15);
-                if (n >= sg.N) continue;
-                const float r = acc[i][j][e] * f;
-                if (blockIdx.z == 0) {
-                    float* p = sg.y + (size_t)t * sg.ldy + n;
-                    *p = a.add ? *p + r : r;
-                } else {
-                    const size_t col = (size_t)(sg.y - a.seg[0].y);
-                    a.part[(size_t)(blockIdx.z - 1) * a.T * sg.ldy + (size_t)t * sg.ldy + col + n] = r;
-                }
-            }
-        }
-}
-
-// launches whose segments are all tile-interleaved Q6_K
-template <int BM>
-__global__ __launch_bounds__(256) void k_pf_gemm_q6k(const PfGemm a) {
-    extern __shared__ __attribute__((aligned(16))) _Float16 pf_ld6[];
-    int bx = blockIdx.x;
-    const int si = pf_seg_of(a, bx);
-    pf_gemm_tile_q6k<BM>(a, a.seg[si], bx * PF_BN, blockIdx.y * BM, pf_ld6);
-}
-
-// launches of tile-interleaved Q4_K and Q6_K segments (q, k in Q4_K, v in Q6_K): each workgroup
-// takes its segment's form
-template <int BM>
-__global__ __launch_bounds__(256) void k_pf_gemm_q46(const PfGemm a) {
-    extern __shared__ __attribute__((aligned(16))) _Float16 pf_ld46[];
-    int bx = blockIdx.x;
-    const int si = pf_seg_of(a, bx);
-    const PfSeg& sg = a.seg[si];
-    if (sg.type == FLLM_TYPE_Q6_K)
-        pf_gemm_tile_q6k<BM>(a, sg, bx * PF_BN, blockIdx.y * BM, pf_ld46);
-    else
-        pf_gemm_tile_q4k<BM>(a, sg, bx * PF_BN, blockIdx.y * BM, pf_ld46);
-}
-
-template <int BM>
-__global__ __launch_bounds__(256) void k_pf_gemm_tiles_h(const PfGemm a) {
-    extern __shared__ __attribute__((aligned(16))) _Float16 pf_ldh[];
-    int bx = blockIdx.x;
-    const int si = pf_seg_of(a, bx);
-    const PfSeg& sg = a.seg[si];
-    _Float16* sw = pf_ldh + (size_t)2 * BM * PF_LDH;
-    if (sg.type == FLLM_TYPE_Q6_K)
-        pf_gemm_tile_h<FLLM_TYPE_Q6_K, BM>(a, sg, bx * PF_BN, blockIdx.y * BM, pf_ldh, sw);
-    else if (sg.type == FLLM_TYPE_Q8_0)
-        pf_gemm_tile_h<FLLM_TYPE_Q8_0, BM>(a, sg, bx * PF_BN, blockIdx.y * BM, pf_ldh, sw);
-    else if (sg.type == FLLM_TYPE_Q5_K)
-        pf_gemm_tile_h<FLLM_TYPE_Q5_K, BM>(a, sg, bx * PF_BN, blockIdx.y * BM, pf_ldh, sw);
-    else
-        pf_gemm_tile_h<FLLM_TYPE_Q4_K, BM>(a, sg, bx * PF_BN, blockIdx.y * BM, pf_ldh, sw);
-}
-
-// launches whose segments are all tile-interleaved Q8_0: the exact-integer Q8_0 form uses one weight
-// plane plus the block scales (pf_gemm_lds_q8 bytes instead of pf_gemm_lds_h), so three workgroups
-// share a CU
-template <int BM>
-static constexpr size_t pf_gemm_lds_q8() {
-    return sizeof(_Float16) * (size_t)(2 * BM + PF_BN) * PF_LDH + sizeof(float) * 2 * PF_BN;
-}
-template <int BM>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void k_pf_gemm_q8t(const PfGemm a) {
-    extern __shared__ __attribute__((aligned(16))) _Float16 pf_ld8[];
-    int bx = blockIdx.x;
-    const int si = pf_seg_of(a, bx);
-    pf_gemm_tile_h<FLLM_TYPE_Q8_0, BM>(a, a.seg[si], bx * PF_BN, blockIdx.y * BM, pf_ld8, pf_ld8 + (size_t)2 * BM * PF_LDH);
-}
-
-// launches whose segments are all tile-interleaved Q5_K
-template <int BM>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(BM == 64 ? 3 : 1))) void k_pf_gemm_q5k(const PfGemm a) {
-    extern __shared__ __attribute__((aligned(16))) _Float16 pf_ld5[];
-    int bx = blockIdx.x;
-    const int si = pf_seg_of(a, bx);
-    pf_gemm_tile_q4k<BM, FLLM_TYPE_Q5_K>(a, a.seg[si], bx * PF_BN, blockIdx.y * BM, pf_ld5);
-}
-
-// launches whose segments are all tile-interleaved Q4_K
-template <int BM>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(BM == 64 ? 3 : 1))) void k_pf_gemm_q4k(const PfGemm a) {
-    extern __shared__ __attribute__((aligned(16))) _Float16 pf_ldk[];
-    int bx = blockIdx.x;
-    const int si = pf_seg_of(a, bx);
-    pf_gemm_tile_q4k<BM>(a, a.seg[si], bx * PF_BN, blockIdx.y * BM, pf_ldk);
 }
 
 template <int BM, int RT>
@@ -1379,8 +634,6 @@ int pf_wexp(unsigned max_bits) {
     return e < -120 ? -120 : (e > 120 ? 120 : e);
 }
 
-typedef void (*PfGemmKernel)(const PfGemm);
-
 // y[i] += part[0][i] + part[1][i] + ... (in that order) over n = T * ldy values
 __global__ __launch_bounds__(256) void k_pf_split_add(float* __restrict__ y, const float* __restrict__ part, int nsp,
                                                       int64_t n) {
@@ -1425,16 +678,16 @@ static hipError_t pf_lds_attr(const void* k, size_t bytes) {
     return hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
 }
 
-// resident workgroups of 256 threads per CU for a GEMM kernel at its LDS size (asked once per kernel)
-static int pf_resident(PfGemmKernel k, size_t lds) {
+// resident workgroups per CU for a GEMM kernel at its LDS size (asked once per kernel)
+static int pf_resident(const PfKernel& k) {
     static std::mutex mu;
     static std::vector<std::pair<PfGemmKernel, int>> seen;
     std::lock_guard<std::mutex> lock(mu);
     for (const auto& e : seen)
-        if (e.first == k) return e.second;
+        if (e.first == k.k) return e.second;
     int per_cu = 0;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, (const void*)k, 256, lds) != hipSuccess) per_cu = 0;
-    seen.emplace_back(k, per_cu);
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, (const void*)k.k, k.threads, k.lds) != hipSuccess) per_cu = 0;
+    seen.emplace_back(k.k, per_cu);
     return per_cu;
 }
 
@@ -1442,108 +695,80 @@ hipError_t launch_pf_gemm(PfGemm a, int n_cu, hipStream_t st, int* pending) {
     if (pending) *pending = 0;
     if (a.T <= 0 || a.nseg <= 0) return hipSuccess;
     if (a.nseg > 3 || a.K <= 0 || a.K % 32 != 0 || a.ldx < a.K || a.ldx % 4 != 0) return hipErrorInvalidValue;
+    if (a.xh == nullptr || a.ldh < a.K || a.ldh % 8 != 0 || a.xs == nullptr) return hipErrorInvalidValue;
     const bool tiles = a.seg[0].layout == LAYOUT_TILES;
-    int64_t col_tiles = 0;
+    int form = tiles ? a.seg[0].type : -1;
     for (int i = 0; i < a.nseg; i++) {
-        PfSeg& g = a.seg[i];
+        const PfSeg& g = a.seg[i];
         if (g.N <= 0 || g.ldy < g.N || (g.layout == LAYOUT_TILES) != tiles) return hipErrorInvalidValue;
         if (!tiles && g.type != a.seg[0].type) return hipErrorInvalidValue;  // one decoder per row launch
         if (tiles && (a.K % 256 != 0 || g.N % 16 != 0 ||
                       (g.type != FLLM_TYPE_Q4_K && g.type != FLLM_TYPE_Q6_K && g.type != FLLM_TYPE_Q8_0 &&
                        g.type != FLLM_TYPE_Q5_K)))
             return hipErrorInvalidValue;
-        g.tiles = (g.N + PF_BN - 1) / PF_BN;
-        col_tiles += g.tiles;
+        if (tiles && g.type != form) form = PF_FORM_MIX;
     }
-    // 64-token tiles at every length: two or three workgroups per CU against one for 128-token
-    // tiles (at 288-352 registers), which ran 15-25% slower even on 4096-token chunks
-    PfGemmKernel k;
-    size_t lds;
-    if (a.xh) {
-        if (a.ldh < a.K || a.ldh % 8 != 0 || a.xs == nullptr) return hipErrorInvalidValue;
-        bool all_q4k = tiles;
-        for (int i = 0; i < a.nseg; i++) all_q4k = all_q4k && a.seg[i].type == FLLM_TYPE_Q4_K;
-        bool all_q6k = tiles, all_q5k = tiles, q46 = tiles, all_q8 = tiles;
-        for (int i = 0; i < a.nseg; i++) {
-            all_q8 = all_q8 && a.seg[i].type == FLLM_TYPE_Q8_0;
-            all_q6k = all_q6k && a.seg[i].type == FLLM_TYPE_Q6_K;
-            all_q5k = all_q5k && a.seg[i].type == FLLM_TYPE_Q5_K;
-            q46 = q46 && (a.seg[i].type == FLLM_TYPE_Q4_K || a.seg[i].type == FLLM_TYPE_Q6_K);
-        }
-        if (all_q4k) {
-            k = k_pf_gemm_q4k<64>;
-            lds = pf_gemm_lds_k<64>();
-        } else if (all_q5k) {
-            k = k_pf_gemm_q5k<64>;
-            lds = pf_gemm_lds_k<64>();
-        } else if (all_q6k) {
-            k = k_pf_gemm_q6k<64>;
-            lds = pf_gemm_lds_q6<64>();
-        } else if (all_q8) {
-            k = k_pf_gemm_q8t<64>;
-            lds = pf_gemm_lds_q8<64>();
-        } else if (q46) {
-            k = k_pf_gemm_q46<64>;
-            lds = std::max(pf_gemm_lds_k<64>(), pf_gemm_lds_q6<64>());
-        } else {
-            if (tiles) k = k_pf_gemm_tiles_h<64>;
-            else k = pf_rows_kernel_h<64>(a.seg[0].type);
-            lds = pf_gemm_lds_h<64>();
-        }
-    } else {
-        return hipErrorInvalidValue;  // the fp16 planes are required
-    }
-    hipError_t e = pf_lds_attr((const void*)k, lds);
-    if (e != hipSuccess) return e;
-    constexpr int bm = 64;
     // K split: a launch whose segments fill the rows of one buffer side by side may run its K in
     // nsplit parts of whole 256-element blocks (part 0 into y, parts z > 0 into the scratch, then a
-    // reduction in order). The choice minimises waves of resident workgroups x blocks per part
-    // plus the reduction's bytes, in units of one block of one full wave: about 0.0118 us per
-    // resident workgroup slot (a 64 x 128 tile's fp16 products at the forms' measured rate), the
-    // reduction reading the parts and y and writing y at 4 TB/s. Llama-3-8B at 511 tokens: o 256
-    // tiles in 3 parts on 768 slots, down 256 in 2 on 512, q/k/v 384 in 4; Qwen2-7B at 2047 tokens:
-    // down 896 tiles in 4 on 768.
+    // reduction in order).
+    bool side_by_side = a.part != nullptr && a.K % 256 == 0;
+    int64_t off = 0;
+    for (int i = 0; i < a.nseg; i++) {
+        const PfSeg& g = a.seg[i];
+        side_by_side = side_by_side && g.ldy == a.seg[0].ldy && g.y - a.seg[0].y == off;
+        off += g.N;
+    }
+    side_by_side = side_by_side && off == a.seg[0].ldy;
+    const double out_bytes = 4.0 * (double)a.T * (double)a.seg[0].ldy;
+    const int cus = n_cu > 0 ? n_cu : 256, nb = a.K / 256;
+    // The kernel and the number of parts of least time: waves of resident workgroups x (blocks per part
+    // x the kernel's time per block + PF_WAVE_US for a workgroup's first loads and last stores), plus the
+    // reduction reading the parts and y and writing y at 4 TB/s. Measured (Q4_K, 28672 x 4096): 511
+    // tokens 281 us on 448 tiles of 128 tokens, 346 on 896 of 64; 37 tokens 47 us on 112 tiles of 64 in
+    // 2 parts, 57 on the 64 x 128 tiles of four waves that these kernels replaced.
+    constexpr double PF_WAVE_US = 4.0;
+    PfKernel k{};
     int nsplit = 1, nbk = 0;
-    if (a.part != nullptr && a.K % 256 == 0) {
-        const int64_t base = col_tiles * ((a.T + bm - 1) / bm);
-        bool side_by_side = true;
-        int64_t off = 0;
-        for (int i = 0; i < a.nseg; i++) {
-            const PfSeg& g = a.seg[i];
-            side_by_side = side_by_side && g.ldy == a.seg[0].ldy && g.y - a.seg[0].y == off;
-            off += g.N;
-        }
-        side_by_side = side_by_side && off == a.seg[0].ldy;
-        const int per_cu = side_by_side ? pf_resident(k, lds) : 0;
-        if (per_cu > 0) {
-            const int64_t slots = (int64_t)per_cu * (n_cu > 0 ? n_cu : 256);
-            const int nb = a.K / 256;
-            const double out_bytes = 4.0 * (double)a.T * (double)a.seg[0].ldy;
-            const double unit_us = 0.0118 * (double)slots;  // one block of one full wave
-            double best = 0.0;
-            // grids of three or more waves unsplit (there the last wave's share is small and the
-            // reduction's cost was not repaid: Gemma-2-9B's o at 4096 tokens ran 6% longer in 2 parts)
-            const int nmax = (base + slots - 1) / slots <= 2 ? 4 : 1;
-            for (int n = 1; n <= nmax && n <= nb; n++) {
-                if (n > 1 && (size_t)(n - 1) * (size_t)a.T * (size_t)a.seg[0].ldy > a.part_cap) break;
-                const int64_t waves = (base * n + slots - 1) / slots;
-                const int bpp = (nb + n - 1) / n;
-                if ((n - 1) * bpp >= nb) continue;  // every part holds at least one block
-                const double cost = (double)waves * bpp + (n > 1 ? (n + 1) * out_bytes / 4.0e6 / unit_us : 0.0);
-                if (n == 1 || cost < best) {
-                    best = cost;
-                    nsplit = n;
-                    nbk = bpp;
-                }
+    int64_t col_tiles = 0;
+    double best = 0.0;
+    for (int c = 0; c < (tiles ? 2 : 1); c++) {
+        PfKernel kc = tiles ? pf_gemm8_kernel(form, c == 0 ? 64 : 128)
+                            : PfKernel{pf_rows_kernel_h<64>(a.seg[0].type), pf_gemm_lds_h<64>(), 64, PF_BN, 256, 0.0};
+        if (kc.k == nullptr) return hipErrorInvalidValue;
+        hipError_t e = pf_lds_attr((const void*)kc.k, kc.lds);
+        if (e != hipSuccess) return e;
+        int64_t ct = 0;
+        for (int i = 0; i < a.nseg; i++) ct += (a.seg[i].N + kc.bn - 1) / kc.bn;
+        const int64_t base = ct * ((a.T + kc.bm - 1) / kc.bm);
+        const int per_cu = tiles ? 1 : pf_resident(kc);
+        const int64_t slots = (int64_t)(per_cu > 0 ? per_cu : 1) * cus;
+        // the row kernels: about 0.0118 us per resident slot and block
+        const double block_us = tiles ? kc.block_us : 0.0118 * (double)slots;
+        // grids of three or more waves unsplit (there the last wave's share is small and the
+        // reduction's cost was not repaid: Gemma-2-9B's o at 4096 tokens ran 6% longer in 2 parts)
+        const int nmax = side_by_side && per_cu > 0 && (base + slots - 1) / slots <= 2 ? (tiles ? 16 : 4) : 1;
+        for (int n = 1; n == 1 || (n <= nmax && n <= nb); n++) {
+            if (n > 1 && (size_t)(n - 1) * (size_t)a.T * (size_t)a.seg[0].ldy > a.part_cap) break;
+            const int64_t waves = (base * n + slots - 1) / slots;
+            const int bpp = ((nb > 0 ? nb : 1) + n - 1) / n;
+            if (n > 1 && (n - 1) * bpp >= nb) continue;  // every part holds at least one block
+            const double cost = (double)waves * (bpp * block_us + (tiles ? PF_WAVE_US : 0.0)) +
+                                (n > 1 ? (n + 1) * out_bytes / 4.0e6 : 0.0);
+            if (k.k == nullptr || cost < best) {
+                best = cost;
+                k = kc;
+                nsplit = n;
+                nbk = bpp;
+                col_tiles = ct;
             }
         }
     }
+    for (int i = 0; i < a.nseg; i++) a.seg[i].tiles = (a.seg[i].N + k.bn - 1) / k.bn;
     a.nsplit = nsplit;
     a.kpart = nsplit > 1 ? 256 * nbk : a.K;
-    dim3 grid((unsigned)col_tiles, (unsigned)((a.T + bm - 1) / bm), (unsigned)nsplit);
-    k<<<grid, 256, lds, st>>>(a);
-    e = hipGetLastError();
+    dim3 grid((unsigned)col_tiles, (unsigned)((a.T + k.bm - 1) / k.bm), (unsigned)nsplit);
+    k.k<<<grid, k.threads, k.lds, st>>>(a);
+    const hipError_t e = hipGetLastError();
     if (e != hipSuccess || nsplit == 1) return e;
     if (pending) {
         *pending = nsplit - 1;

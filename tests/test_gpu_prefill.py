@@ -12,7 +12,7 @@ import pytest
 import dotnetfoundryllm_amd as F
 import dotnetfoundryllm_amd._native as N
 import oracle_bind as O
-from dotnetfoundryllm_amd.configs import desc_of, synth_bytes, tensor_plan
+from dotnetfoundryllm_amd.configs import CONFIGS, desc_of, synth_bytes, tensor_plan
 from fixtures import synthetic, upload
 
 pytestmark = pytest.mark.gpu
@@ -283,5 +283,49 @@ def test_prefill_argument_contract(ctx):
         with pytest.raises(F.ArgumentOutOfRangeException):
             fwd.prefill(np.array([1, 2], dtype=np.int32), 16, kv)  # cache full
     finally:
+        kv.close()
+        m.close()
+
+
+@pytest.mark.parametrize("types", [("q4_k",) * 7, ("q5_k",) * 7, ("q6_k",) * 7, ("q8_0",) * 7,
+                                   ("q5_k", "q8_0", "q6_k", "q4_k", "q4_k", "q6_k", "q5_k")],
+                         ids=["q4_k", "q5_k", "q6_k", "q8_0", "mixed"])
+def test_prefill_gemm_tile_edges(ctx, types):
+    """The tile-interleaved GEMMs at the edges of their tiles (64 and 128 tokens x 256 weight rows):
+    1 to 200 tokens on 128-, 512- and 768-row matrices of 2 and 3 blocks, every tile type alone and
+    launches that mix them. K / V rows of both layers (the second layer's carry every GEMM of the
+    first) against the oracle. Bound: operands of 22 bits or more and f32 sums of at most 768
+    products, 2^-22 + sqrt(768) 2^-24 (2e-6) for a projection, five of them in a row: 1e-5; twice that.
+    The softmax multiplies a score's relative error by the score, and these seeded weights make
+    scores q k of about 5e4 (|q|, |k| about 27 over 64 elements): Gemma-2's own attention scale, here
+    1e-5, keeps the scores below 1 and the bound that of the GEMMs. It is the median row's; a row whose
+    sums nearly cancel (the seeded weights are not zero-mean) has the file's bar."""
+    name_of = {"q4_k": N.Q4_K, "q5_k": N.Q5_K, "q6_k": N.Q6_K, "q8_0": N.Q8_0}
+    t = [name_of[x] for x in types]
+    cfg = dict(CONFIGS["test-gemma2"], n_layers=2, hidden=512, n_heads=8, n_kv_heads=2, head_dim=64, ffn=768, max_ctx=256,
+               window=0x7FFFFFFF,
+               types=dict(zip(("q", "k", "v", "o", "gate", "up", "down", "out"), t + [t[0]])))
+    desc = desc_of(cfg)
+    desc.attn_scale = 1e-5
+    tensors = {e[0]: (e, synth_bytes(cfg, e)) for e in tensor_plan(cfg)}
+    m = device_model(ctx, desc, tensors)
+    kv, fwd = F.HipKvCache(m), F.HipForwardPass(m)
+    orc = O.OracleModel(desc, tensors)
+    prompt = F.synth_tokens(cfg["seed"], 9, desc.vocab, 200)
+    try:
+        _oracle_prefill(orc, prompt)
+        for n in (2, 33, 64, 65, 128, 129, 200):
+            kv.clear()
+            fwd.prefill(prompt[:n], 0, kv)
+            for l in range(desc.n_layers):
+                for kind, get in ((0, kv.get_keys), (1, kv.get_values)):
+                    got, want = get(l), orc.kv(l, kind)
+                    got = np.asarray(got, dtype=np.float64).reshape(n, -1)
+                    want = np.asarray(want, dtype=np.float64).reshape(-1)[:got.size].reshape(n, -1)
+                    err = np.linalg.norm(got - want, axis=1) / np.linalg.norm(want, axis=1)
+                    assert np.median(err) <= 2e-5 and err.max() <= TOL, (n, l, kind, err.max())
+        assert O.normwise_rel_err(fwd.logits, orc.logits()) <= TOL
+    finally:
+        orc.close()
         kv.close()
         m.close()
