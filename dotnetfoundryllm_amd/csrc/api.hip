@@ -1684,7 +1684,7 @@ struct PfSrc {
     const float* w;
     float eps;
     int fn;       // NORM: 1 GemmaRmsNorm; ACT: 1 GELU, 0 SiLU
-    int nsp = 0;  // NORM: K-split slices of x left in pf_part by the previous GEMM, added into x first
+    int nsp = 0;  // K-split slices of x left in pf_part by the previous GEMM, added first (NORM: into x)
 };
 
 // y_i (+)= X W_i^T over the chunk's rows for the matrices w[0..n) (one launch when their layouts
@@ -1715,8 +1715,8 @@ static hipError_t pf_gemm(fllm_seq* s, const char* name, const Tensor* const* w,
     } else if (src && src->kind == PfSrc::ACT) {
         g.x = src->x;
         g.ldx = 2 * g.K;
-        STEP("pf_act_split", 8.0 * T * g.K + 4.0 * T * g.ldh,
-             launch_pf_split_act(src->x, T, g.K, src->fn, s->pf_xh, g.ldh, s->pf_xs, s->st));
+        STEP("pf_act_split", (8.0 + 8.0 * src->nsp) * T * g.K + 4.0 * T * g.ldh,
+             launch_pf_split_act(src->x, T, g.K, src->fn, s->pf_xh, g.ldh, s->pf_xs, s->st, s->pf_part, src->nsp));
     } else {
         STEP("pf_split", 4.0 * T * g.K + 4.0 * T * g.ldh,
              launch_pf_split(g.x, g.ldx, T, g.K, s->pf_xh, g.ldh, s->pf_xs, s->st));
@@ -1800,20 +1800,21 @@ static hipError_t prefill_chunk(fllm_seq* s, int T, int pos0) {
                      launch_pf_postnorm_add(s->pf_tmp, T, H, L.post_attn, s->pf_x, s->st, s->pf_part, pend_t));
         }
         if (!fuse_h) STEP("pf_norm", 8.0 * T * H, launch_pf_norm(s->pf_x, T, H, L.ffn_norm, eps, nk, s->pf_xn, ldx, s->st));
+        int pend_gu = 0;
         {
             const Tensor* w[2] = {&L.gate, &L.up};
             float* y[2] = {s->pf_gu, s->pf_gu + F};
             const PfSrc src{PfSrc::NORM, s->pf_x, L.ffn_norm, eps, nk, pend_x};
             pend_x = 0;
-            if ((e = pf_gemm(s, "pf_gate_up", w, y, 2, 2 * F, T, false, nullptr, 0, fuse_h ? &src : nullptr)) !=
-                hipSuccess)
+            if ((e = pf_gemm(s, "pf_gate_up", w, y, 2, 2 * F, T, false, nullptr, 0, fuse_h ? &src : nullptr,
+                             fuse_f ? &pend_gu : nullptr)) != hipSuccess)
                 return e;
         }
         if (!fuse_f) STEP("pf_act", 12.0 * T * F, launch_pf_act(s->pf_gu, T, F, gemma ? 1 : 0, s->pf_xn, ldx, s->st));
         {
             const Tensor* w[1] = {&L.down};
             float* y[1] = {gemma ? s->pf_tmp : s->pf_x};
-            const PfSrc src{PfSrc::ACT, s->pf_gu, nullptr, 0.0f, gemma ? 1 : 0};
+            const PfSrc src{PfSrc::ACT, s->pf_gu, nullptr, 0.0f, gemma ? 1 : 0, pend_gu};
             // the last layer's sum is complete when the chunk ends; Gemma-2's goes into the post-norm
             int pend_t = 0;
             if ((e = pf_gemm(s, "pf_down", w, y, 1, H, T, !gemma, nullptr, 0, fuse_f ? &src : nullptr,

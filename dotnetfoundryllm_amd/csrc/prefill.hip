@@ -28,6 +28,7 @@
 namespace fllm {
 
 typedef float pf_f32x4 __attribute__((ext_vector_type(4)));
+typedef float pf_f32x2 __attribute__((ext_vector_type(2)));
 
 __device__ __forceinline__ float pf_wave_sum(float v) {
 #pragma unroll
@@ -39,12 +40,34 @@ __device__ __forceinline__ float pf_wave_max(float v) {
     for (int o = 32; o > 0; o >>= 1) v = fmaxf(v, __shfl_xor(v, o));
     return v;
 }
-// sum over a 256-thread workgroup (called once per kernel by every thread)
+// sum over a workgroup of NW waves, 4 or 16 (called once per kernel by every thread)
+template <int NW = 4>
 __device__ __forceinline__ float pf_block_sum(float v, float* red) {
     v = pf_wave_sum(v);
     if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
     __syncthreads();
+    if constexpr (NW == 16) {
+        v = 0.0f;
+#pragma unroll
+        for (int i = 0; i < 16; i += 4) v += (red[i] + red[i + 1]) + (red[i + 2] + red[i + 3]);
+        return v;
+    }
     return (red[0] + red[1]) + (red[2] + red[3]);
+}
+// v += p[0] + p[pn] + ... + p[(nsp - 1) pn] in that order, four loads in flight (a K-split launch leaves
+// up to 15 slices, and one load at a time waits a memory latency each)
+template <typename V>
+__device__ __forceinline__ V pf_add_slices(V v, const float* __restrict__ p, int nsp, size_t pn) {
+    int z = 0;
+    for (; z + 4 <= nsp; z += 4) {
+        V q[4];
+#pragma unroll
+        for (int u = 0; u < 4; u++) q[u] = *(const V*)(p + (size_t)(z + u) * pn);
+#pragma unroll
+        for (int u = 0; u < 4; u++) v += q[u];
+    }
+    for (; z < nsp; z++) v += *(const V*)(p + (size_t)z * pn);
+    return v;
 }
 // LDS written by lanes of a wave, then read by other lanes of the same wave
 __device__ __forceinline__ void pf_wave_sync() {
@@ -447,72 +470,82 @@ __global__ __launch_bounds__(256) void k_pf_split(const float* __restrict__ x, i
     if (threadIdx.x == 0) xs[t] = ldexpf(1.0f, -e);
 }
 
+template <int SRC>
+static hipError_t pf_split_src(float* x, int ldx, int T, int K, const float* w, float eps, int kind,
+                               _Float16* xh, int ldh, float* xs, hipStream_t st, const float* part, int nsp);
 hipError_t launch_pf_split(const float* x, int ldx, int T, int K, _Float16* xh, int ldh, float* xs, hipStream_t st) {
     if (T <= 0) return hipSuccess;
     if (K % 32 != 0 || ldx % 4 != 0 || ldh % 8 != 0 || ldh < K) return hipErrorInvalidValue;
+    // rows that fit in registers are read once (the form without weights only reads x)
+    if (pf_split_src_ok(K))
+        return pf_split_src<0>(const_cast<float*>(x), ldx, T, K, nullptr, 0.0f, 0, xh, ldh, xs, st, nullptr, 0);
     k_pf_split<<<T, 256, 0, st>>>(x, ldx, K, xh, ldh, (size_t)T * ldh, xs, T);
     return hipGetLastError();
 }
 
-// The split of a row computed here rather than read: SRC 1, RmsNorm / GemmaRmsNorm (kind 1) of row
-// t of x (row stride ldx, weights w), k_pf_norm's arithmetic per element; SRC 2, act(gate) * up of row
-// t of gu (gate in columns [0, K), up in [K, 2 K) of a row of stride ldx), k_pf_act's. The row stays
-// in registers (NPT float4 per thread: element 4 i .. 4 i + 3 with i = thread + 256 j), so the
-// normalized or gated row is never written; the scale, planes and group sums are k_pf_split's.
-// SRC 1 with nsp > 0: the row is x[t] + part[0][t] + ... + part[nsp - 1][t] (slices of pn floats,
-// row stride ldx), k_pf_split_add's sum, written back to x before the norm.
-template <int NPT, int SRC>
-__global__ __launch_bounds__(256) void k_pf_split_src(float* __restrict__ x, int ldx, int K,
-                                                      const float* __restrict__ w, float eps, int kind,
-                                                      _Float16* __restrict__ xh, int ldh, size_t plane,
-                                                      float* __restrict__ xs, int T, const float* __restrict__ part,
-                                                      int nsp, size_t pn) {
-    __shared__ float red[4];
+// The split of a row: SRC 0, row t of x (row stride ldx) as it is; SRC 1, its RmsNorm / GemmaRmsNorm
+// (kind 1, weights w), k_pf_norm's arithmetic per element; SRC 2, act(gate) * up of row t of gu (gate in
+// columns [0, K), up in [K, 2 K) of a row of stride ldx), k_pf_act's. The row stays in registers (NPT
+// float4 per thread: element 4 i .. 4 i + 3 with i = thread + 64 NW j), so the normalized or gated row is
+// never written; the scale, planes and group sums are k_pf_split's. SRC 1 and 2 with nsp > 0: the row is
+// x[t] + part[0][t] + ... + part[nsp - 1][t] (slices of pn floats, row stride ldx), k_pf_split_add's
+// sum; SRC 1 writes it back to x.
+// One workgroup of NW waves per row. 37 rows of 4096 with 15 slices: 16.0 us with 4 waves and one slice
+// load at a time, 6.4 with 16 waves and four.
+// rows up to which a row-wise kernel spreads each row over 16 waves (two rows per CU)
+constexpr int PF_FEW_ROWS = 512;
+template <int NPT, int SRC, int NW>
+__global__ __launch_bounds__(64 * NW) void k_pf_split_src(float* __restrict__ x, int ldx, int K,
+                                                          const float* __restrict__ w, float eps, int kind,
+                                                          _Float16* __restrict__ xh, int ldh, size_t plane,
+                                                          float* __restrict__ xs, int T, const float* __restrict__ part,
+                                                          int nsp, size_t pn) {
+    constexpr int NT = 64 * NW;
+    __shared__ float red[NW];
     const int t = blockIdx.x;
     float* xr = x + (size_t)t * ldx;
+    const float* pr = part + (size_t)t * ldx;
     const int K4 = K / 4;
-    float4 v[NPT];
+    pf_f32x4 v[NPT];
     float ss = 0.0f;
 #pragma unroll
     for (int j = 0; j < NPT; j++) {
-        const int i = threadIdx.x + 256 * j;
-        float4 q = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+        const int i = threadIdx.x + NT * j;
+        pf_f32x4 q = {0.0f, 0.0f, 0.0f, 0.0f};
         if (i < K4) {
+            q = ((const pf_f32x4*)xr)[i];
             if constexpr (SRC == 2) {
-                const float4 g = ((const float4*)xr)[i], u = ((const float4*)(xr + K))[i];
-                q = make_float4(act_fn(g.x, kind) * u.x, act_fn(g.y, kind) * u.y, act_fn(g.z, kind) * u.z,
-                                act_fn(g.w, kind) * u.w);
-            } else {
-                q = ((const float4*)xr)[i];
+                pf_f32x4 u = ((const pf_f32x4*)(xr + K))[i];
                 if (nsp > 0) {
-                    for (int z = 0; z < nsp; z++) {
-                        const float4 p = ((const float4*)(part + (size_t)z * pn + (size_t)t * ldx))[i];
-                        q.x += p.x;
-                        q.y += p.y;
-                        q.z += p.z;
-                        q.w += p.w;
-                    }
-                    ((float4*)xr)[i] = q;
+                    q = pf_add_slices(q, pr + 4 * i, nsp, pn);
+                    u = pf_add_slices(u, pr + K + 4 * i, nsp, pn);
                 }
-                ss = fmaf(q.x, q.x, ss);
-                ss = fmaf(q.y, q.y, ss);
-                ss = fmaf(q.z, q.z, ss);
-                ss = fmaf(q.w, q.w, ss);
+#pragma unroll
+                for (int e = 0; e < 4; e++) q[e] = act_fn(q[e], kind) * u[e];
+            } else if constexpr (SRC == 1) {
+                if (nsp > 0) {
+                    q = pf_add_slices(q, pr + 4 * i, nsp, pn);
+                    ((pf_f32x4*)xr)[i] = q;
+                }
+#pragma unroll
+                for (int e = 0; e < 4; e++) ss = fmaf(q[e], q[e], ss);
             }
         }
         v[j] = q;
     }
     if constexpr (SRC == 1) {
-        const float tot = pf_block_sum(ss, red);
+        const float tot = pf_block_sum<NW>(ss, red);
         const float rms = 1.0f / sqrtf(tot / (float)K + eps);
 #pragma unroll
         for (int j = 0; j < NPT; j++) {
-            const int i = threadIdx.x + 256 * j;
+            const int i = threadIdx.x + NT * j;
             if (i < K4) {
-                const float4 w4 = ((const float4*)w)[i];
-                const float t0 = v[j].x * rms, t1 = v[j].y * rms, t2 = v[j].z * rms, t3 = v[j].w * rms;
-                v[j] = kind ? make_float4(t0 * (w4.x + 1.0f), t1 * (w4.y + 1.0f), t2 * (w4.z + 1.0f), t3 * (w4.w + 1.0f))
-                            : make_float4(t0 * w4.x, t1 * w4.y, t2 * w4.z, t3 * w4.w);
+                const pf_f32x4 w4 = ((const pf_f32x4*)w)[i];
+#pragma unroll
+                for (int e = 0; e < 4; e++) {
+                    const float tv = v[j][e] * rms;
+                    v[j][e] = kind ? tv * (w4[e] + 1.0f) : tv * w4[e];
+                }
             }
         }
         __syncthreads();  // red is reused below
@@ -520,11 +553,13 @@ __global__ __launch_bounds__(256) void k_pf_split_src(float* __restrict__ x, int
     float m = 0.0f;
 #pragma unroll
     for (int j = 0; j < NPT; j++)
-        m = fmaxf(m, fmaxf(fmaxf(fabsf(v[j].x), fabsf(v[j].y)), fmaxf(fabsf(v[j].z), fabsf(v[j].w))));
+        m = fmaxf(m, fmaxf(fmaxf(fabsf(v[j][0]), fabsf(v[j][1])), fmaxf(fabsf(v[j][2]), fabsf(v[j][3]))));
     m = pf_wave_max(m);
     if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = m;
     __syncthreads();
-    m = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
+    m = red[0];
+#pragma unroll
+    for (int i = 1; i < NW; i++) m = fmaxf(m, red[i]);
     int e = 0;
     if (m > 0.0f && m <= 3.0e38f) {
         int ex;
@@ -539,8 +574,8 @@ __global__ __launch_bounds__(256) void k_pf_split_src(float* __restrict__ x, int
     const size_t gplane = (size_t)T * G;
 #pragma unroll
     for (int j = 0; j < NPT; j++) {
-        const int i = threadIdx.x + 256 * j;
-        const float c[4] = {v[j].x * sc, v[j].y * sc, v[j].z * sc, v[j].w * sc};
+        const int i = threadIdx.x + NT * j;
+        const float c[4] = {v[j][0] * sc, v[j][1] * sc, v[j][2] * sc, v[j][3] * sc};
         if (i < K4) {
             _Float16 hi[4], lo[4];
 #pragma unroll
@@ -568,24 +603,32 @@ __global__ __launch_bounds__(256) void k_pf_split_src(float* __restrict__ x, int
 
 template <int SRC>
 static hipError_t pf_split_src(float* x, int ldx, int T, int K, const float* w, float eps, int kind,
-                               _Float16* xh, int ldh, float* xs, hipStream_t st, const float* part = nullptr,
-                               int nsp = 0) {
+                               _Float16* xh, int ldh, float* xs, hipStream_t st, const float* part, int nsp) {
     if (T <= 0) return hipSuccess;
     if (K % 32 != 0 || ldx % 4 != 0 || ldh % 8 != 0 || ldh < K) return hipErrorInvalidValue;
-    if (nsp < 0 || (nsp > 0 && (SRC != 1 || part == nullptr || (uintptr_t)part % 16 != 0))) return hipErrorInvalidValue;
-    const int n4 = (K / 4 + 255) / 256;
+    if (nsp < 0 || (nsp > 0 && (SRC == 0 || part == nullptr || (uintptr_t)part % 16 != 0))) return hipErrorInvalidValue;
     const size_t plane = (size_t)T * ldh, pn = (size_t)T * ldx;
-    if (n4 <= 1) k_pf_split_src<1, SRC><<<T, 256, 0, st>>>(x, ldx, K, w, eps, kind, xh, ldh, plane, xs, T, part, nsp, pn);
-    else if (n4 <= 2) k_pf_split_src<2, SRC><<<T, 256, 0, st>>>(x, ldx, K, w, eps, kind, xh, ldh, plane, xs, T, part, nsp, pn);
-    else if (n4 <= 4) k_pf_split_src<4, SRC><<<T, 256, 0, st>>>(x, ldx, K, w, eps, kind, xh, ldh, plane, xs, T, part, nsp, pn);
-    else if (n4 <= 8) k_pf_split_src<8, SRC><<<T, 256, 0, st>>>(x, ldx, K, w, eps, kind, xh, ldh, plane, xs, T, part, nsp, pn);
-    else if (n4 <= 16) k_pf_split_src<16, SRC><<<T, 256, 0, st>>>(x, ldx, K, w, eps, kind, xh, ldh, plane, xs, T, part, nsp, pn);
-    else if (n4 <= 20) k_pf_split_src<20, SRC><<<T, 256, 0, st>>>(x, ldx, K, w, eps, kind, xh, ldh, plane, xs, T, part, nsp, pn);
+    if (nsp == 0) part = x;  // not read
+    auto run = [&](auto kern, int threads) {
+        kern<<<T, threads, 0, st>>>(x, ldx, K, w, eps, kind, xh, ldh, plane, xs, T, part, nsp, pn);
+    };
+    // 16 waves per row while the rows leave the chip idle (T <= PF_FEW_ROWS), 4 above: at 4096 rows of
+    // 3584 the norm form measured 24.3 us with 4 waves and 28.6 with 16, at 37 rows 8.3 and 6.4
+    const int n4 = K / 4;
+    const bool wide = T <= PF_FEW_ROWS;
+    if (n4 <= 256) run(k_pf_split_src<1, SRC, 4>, 256);
+    else if (n4 <= 512) run(k_pf_split_src<2, SRC, 4>, 256);
+    else if (n4 <= 1024 && wide) run(k_pf_split_src<1, SRC, 16>, 1024);
+    else if (n4 <= 1024) run(k_pf_split_src<4, SRC, 4>, 256);
+    else if (n4 <= 2048 && wide) run(k_pf_split_src<2, SRC, 16>, 1024);
+    else if (n4 <= 2048) run(k_pf_split_src<8, SRC, 4>, 256);
+    else if (n4 <= 4096) run(k_pf_split_src<4, SRC, 16>, 1024);
+    else if (n4 <= 5120) run(k_pf_split_src<5, SRC, 16>, 1024);
     else return hipErrorNotSupported;
     return hipGetLastError();
 }
 
-bool pf_split_src_ok(int K) { return K % 32 == 0 && (K / 4 + 255) / 256 <= 20; }
+bool pf_split_src_ok(int K) { return K % 32 == 0 && K <= 20480; }
 
 hipError_t launch_pf_split_norm(float* x, int T, int K, const float* w, float eps, int kind, _Float16* xh,
                                 int ldh, float* xs, hipStream_t st, const float* part, int nsp) {
@@ -593,9 +636,9 @@ hipError_t launch_pf_split_norm(float* x, int T, int K, const float* w, float ep
 }
 
 hipError_t launch_pf_split_act(const float* gu, int T, int ffn, int act, _Float16* xh, int ldh, float* xs,
-                               hipStream_t st) {
+                               hipStream_t st, const float* part, int nsp) {
     // the gated form only reads gu
-    return pf_split_src<2>(const_cast<float*>(gu), 2 * ffn, T, ffn, nullptr, 0.0f, act, xh, ldh, xs, st);
+    return pf_split_src<2>(const_cast<float*>(gu), 2 * ffn, T, ffn, nullptr, 0.0f, act, xh, ldh, xs, st, part, nsp);
 }
 
 // largest |w| of a matrix (exact dequantization of every element), as float bits (non-negative floats
@@ -640,17 +683,8 @@ __global__ __launch_bounds__(256) void k_pf_split_add(float* __restrict__ y, con
     // four floats per thread and step where n and the pointers allow (the parts are added in order
     // either way)
     const int64_t n4 = n % 4 == 0 && ((uintptr_t)y | (uintptr_t)part) % 16 == 0 ? n / 4 : 0;
-    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n4; i += (int64_t)gridDim.x * blockDim.x) {
-        float4 v = ((const float4*)y)[i];
-        for (int z = 0; z < nsp; z++) {
-            const float4 w = ((const float4*)(part + (int64_t)z * n))[i];
-            v.x += w.x;
-            v.y += w.y;
-            v.z += w.z;
-            v.w += w.w;
-        }
-        ((float4*)y)[i] = v;
-    }
+    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n4; i += (int64_t)gridDim.x * blockDim.x)
+        ((pf_f32x4*)y)[i] = pf_add_slices(((const pf_f32x4*)y)[i], part + 4 * i, nsp, (size_t)n);
     for (int64_t i = 4 * n4 + (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) {
         float v = y[i];
         for (int z = 0; z < nsp; z++) v += part[(int64_t)z * n + i];
@@ -722,8 +756,8 @@ hipError_t launch_pf_gemm(PfGemm a, int n_cu, hipStream_t st, int* pending) {
     const double out_bytes = 4.0 * (double)a.T * (double)a.seg[0].ldy;
     const int cus = n_cu > 0 ? n_cu : 256, nb = a.K / 256;
     // The kernel and the number of parts of least time: waves of resident workgroups x (blocks per part
-    // x the kernel's time per block + PF_WAVE_US for a workgroup's first loads and last stores), plus the
-    // reduction reading the parts and y and writing y at 4 TB/s. Measured (Q4_K, 28672 x 4096): 511
+    // x the kernel's time per block + PF_WAVE_US for a workgroup's first loads and last stores), plus
+    // writing the parts and reading them in the next kernel at 4 TB/s. Measured (Q4_K, 28672 x 4096): 511
     // tokens 281 us on 448 tiles of 128 tokens, 346 on 896 of 64; 37 tokens 47 us on 112 tiles of 64 in
     // 2 parts, 57 on the 64 x 128 tiles of four waves that these kernels replaced.
     constexpr double PF_WAVE_US = 4.0;
@@ -752,9 +786,11 @@ hipError_t launch_pf_gemm(PfGemm a, int n_cu, hipStream_t st, int* pending) {
             const int64_t waves = (base * n + slots - 1) / slots;
             const int bpp = ((nb > 0 ? nb : 1) + n - 1) / n;
             if (n > 1 && (n - 1) * bpp >= nb) continue;  // every part holds at least one block
+            // a split has to win by 5% (at 4096 tokens, 14336 -> 3584 in 4 parts modelled 3% better and
+            // ran even, its 235 MB of parts slowing the next kernel by 20 us)
             const double cost = (double)waves * (bpp * block_us + (tiles ? PF_WAVE_US : 0.0)) +
-                                (n > 1 ? (n + 1) * out_bytes / 4.0e6 : 0.0);
-            if (k.k == nullptr || cost < best) {
+                                2 * (n - 1) * out_bytes / 4.0e6;
+            if (k.k == nullptr || cost * (n > 1 ? 1.05 : 1.0) < best) {
                 best = cost;
                 k = kc;
                 nsplit = n;
@@ -786,17 +822,26 @@ hipError_t launch_pf_split_add(float* y, const float* part, int nsp, int64_t n, 
 }
 
 // ---- element-wise steps over the rows ----------------------------------------------------------
+// four elements per thread, 1024 per workgroup: a row's loads are all in flight (one workgroup per row had
+// each thread load 16 elements of 4096 one after another: 12.7 us at 37 tokens)
 __global__ __launch_bounds__(256) void k_pf_embed(const int* __restrict__ tok, const uint8_t* __restrict__ emb, int type,
                                                   int H, float* __restrict__ x) {
-    const int t = blockIdx.x;
+    const int t = blockIdx.y, i0 = blockIdx.x * 1024 + threadIdx.x;
     const int64_t base = (int64_t)tok[t] * H;
-    for (int i = threadIdx.x; i < H; i += 256) x[(size_t)t * H + i] = deq_elem(type, emb, base + i);
+    float v[4];
+#pragma unroll
+    for (int u = 0; u < 4; u++) v[u] = i0 + 256 * u < H ? deq_elem(type, emb, base + i0 + 256 * u) : 0.0f;
+#pragma unroll
+    for (int u = 0; u < 4; u++)
+        if (i0 + 256 * u < H) x[(size_t)t * H + i0 + 256 * u] = v[u];
 }
 
 hipError_t launch_pf_embed(const int* tokens, int T, const uint8_t* emb, int type, int H, float* x, hipStream_t st) {
-    if (T <= 0) return hipSuccess;
-    k_pf_embed<<<T, 256, 0, st>>>(tokens, emb, type, H, x);
-    return hipGetLastError();
+    for (int t0 = 0; t0 < T; t0 += 65535) {  // grid.y
+        const int n = T - t0 < 65535 ? T - t0 : 65535;
+        k_pf_embed<<<dim3((unsigned)((H + 1023) / 1024), (unsigned)n), 256, 0, st>>>(tokens + t0, emb, type, H, x + (size_t)t0 * H);
+    }
+    return T > 0 ? hipGetLastError() : hipSuccess;
 }
 
 // RmsNorm (TensorOperations.cs:42-54) / GemmaRmsNorm (:90-107) of row blockIdx.x
@@ -850,43 +895,37 @@ __global__ __launch_bounds__(256) void k_pf_qkv_post(float* __restrict__ qkv, in
     const int t = blockIdx.x, pos = pos0 + t, half = hd >> 1, qdim = nh * hd, kvdim = nkv * hd;
     float* row = qkv + (size_t)t * ldq;
     const float* prow = part + (size_t)t * ldq;
-    // values c, c + 1 (c even; every row, slice and cache row starts at an even offset)
-    auto val2 = [&](int c) {
-        float2 v = *(const float2*)(row + c);
-        for (int z = 0; z < nsp; z++) {
-            const float2 p = *(const float2*)(prow + (size_t)z * pn + c);
-            v.x += p.x;
-            v.y += p.y;
-        }
-        return v;
-    };
-    const float2* rp = rope + (size_t)pos * half;
     const int npairs = (nh + nkv) * half;
-    for (int idx = threadIdx.x; idx < npairs; idx += 256) {
-        const bool isq = idx < nh * half;
-        const int li = isq ? idx : idx - nh * half;
-        const int head = li / half, i = li % half, o = head * hd + 2 * i;
-        const float2 xv = val2((isq ? 0 : qdim) + o);
-        float x0 = xv.x, x1 = xv.y;
-        const float* b = isq ? bq : bk;
-        if (b) {
-            const float2 bb = *(const float2*)(b + o);
-            x0 = x0 + bb.x;
-            x1 = x1 + bb.y;
+    // pairs (c, c + 1) of the row's q, k and v, four per thread and step with their loads together (c
+    // even; every row, slice and cache row starts at an even offset)
+    const int total = npairs + (kvdim >> 1), step = 256 * gridDim.y;
+    for (int i0 = blockIdx.y * 256 + threadIdx.x; i0 < total; i0 += 4 * step) {
+        pf_f32x2 xv[4];
+#pragma unroll
+        for (int u = 0; u < 4; u++)
+            if (i0 + u * step < total) xv[u] = *(const pf_f32x2*)(row + 2 * (i0 + u * step));
+#pragma unroll
+        for (int u = 0; u < 4; u++) {
+            const int idx = i0 + u * step;
+            if (idx >= total) break;
+            xv[u] = pf_add_slices(xv[u], prow + 2 * idx, nsp, pn);
+            float x0 = xv[u][0], x1 = xv[u][1];
+            const int sec = idx < nh * half ? 0 : idx < npairs ? 1 : 2;  // q, k, v
+            const int o = 2 * idx - (sec == 0 ? 0 : sec == 1 ? qdim : qdim + kvdim);
+            const float* b = sec == 0 ? bq : sec == 1 ? bk : bv;
+            if (b) {
+                const float2 bb = *(const float2*)(b + o);
+                x0 = x0 + bb.x;
+                x1 = x1 + bb.y;
+            }
+            if (sec == 2) {
+                *(float2*)(vc + (size_t)pos * kvdim + o) = make_float2(x0, x1);
+            } else {
+                const float2 cs = rope[(size_t)pos * half + ((unsigned)o % (unsigned)hd >> 1)];
+                const float2 y = make_float2(x0 * cs.x - x1 * cs.y, x0 * cs.y + x1 * cs.x);
+                *(float2*)((sec == 0 ? row : kc + (size_t)pos * kvdim) + o) = y;
+            }
         }
-        const float2 cs = rp[i];
-        const float2 y = make_float2(x0 * cs.x - x1 * cs.y, x0 * cs.y + x1 * cs.x);
-        if (isq) *(float2*)(row + o) = y;
-        else *(float2*)(kc + (size_t)pos * kvdim + o) = y;
-    }
-    for (int i = 2 * threadIdx.x; i < kvdim; i += 512) {
-        float2 v = val2(qdim + kvdim + i);
-        if (bv) {
-            const float2 bb = *(const float2*)(bv + i);
-            v.x = v.x + bb.x;
-            v.y = v.y + bb.y;
-        }
-        *(float2*)(vc + (size_t)pos * kvdim + i) = v;
     }
 }
 
@@ -896,7 +935,9 @@ hipError_t launch_pf_qkv_post(float* qkv, int ldq, int T, int pos0, const float*
     if (T <= 0) return hipSuccess;
     if (nsp < 0 || (nsp > 0 && part == nullptr)) return hipErrorInvalidValue;
     if (ldq % 2 != 0 || hd % 2 != 0) return hipErrorInvalidValue;  // pairs of floats at even offsets
-    k_pf_qkv_post<<<T, 256, 0, st>>>(qkv, ldq, pos0, bq, bk, bv, rope, nh, nkv, hd, kc, vc, nsp > 0 ? part : qkv, nsp,
+    // few rows: a pair per thread; many: one workgroup per row (4096 rows: 51 us against 60)
+    const int pairs = (nh + 2 * nkv) * (hd / 2);
+    k_pf_qkv_post<<<dim3((unsigned)T, T <= PF_FEW_ROWS ? (unsigned)((pairs + 255) / 256) : 1u), 256, 0, st>>>(qkv, ldq, pos0, bq, bk, bv, rope, nh, nkv, hd, kc, vc, nsp > 0 ? part : qkv, nsp,
                                      (size_t)T * ldq);
     return hipGetLastError();
 }
@@ -904,40 +945,31 @@ hipError_t launch_pf_qkv_post(float* qkv, int ldq, int T, int pos0, const float*
 // Gemma2 post-norm: x += GemmaRmsNorm(tmp, w), eps 1e-6 (Gemma2ForwardPass.cs:90-96)
 // (n a multiple of 4: float4 pieces; nsp pending K-split slices of part, pn floats apart, added to
 // tmp's row first and written back, k_pf_split_add's sum)
-__global__ __launch_bounds__(256) void k_pf_postnorm_add(float* __restrict__ tmp, int n, const float* __restrict__ w,
-                                                         float* __restrict__ x, const float* __restrict__ part, int nsp,
-                                                         size_t pn) {
-    __shared__ float red[4];
+template <int NW>
+__global__ __launch_bounds__(64 * NW) void k_pf_postnorm_add(float* __restrict__ tmp, int n, const float* __restrict__ w,
+                                                          float* __restrict__ x, const float* __restrict__ part, int nsp,
+                                                          size_t pn) {
+    __shared__ float red[NW];
     const int t = blockIdx.x, n4 = n / 4;
-    float4* tr = (float4*)(tmp + (size_t)t * n);
+    pf_f32x4* tr = (pf_f32x4*)(tmp + (size_t)t * n);
     float ss = 0.0f;
-    for (int i = threadIdx.x; i < n4; i += 256) {
-        float4 v = tr[i];
+    for (int i = threadIdx.x; i < n4; i += 64 * NW) {
+        pf_f32x4 v = tr[i];
         if (nsp > 0) {
-            for (int z = 0; z < nsp; z++) {
-                const float4 p = ((const float4*)(part + (size_t)z * pn + (size_t)t * n))[i];
-                v.x += p.x;
-                v.y += p.y;
-                v.z += p.z;
-                v.w += p.w;
-            }
+            v = pf_add_slices(v, part + (size_t)t * n + 4 * i, nsp, pn);
             tr[i] = v;  // read back below by this same thread
         }
-        ss = fmaf(v.x, v.x, ss);
-        ss = fmaf(v.y, v.y, ss);
-        ss = fmaf(v.z, v.z, ss);
-        ss = fmaf(v.w, v.w, ss);
+#pragma unroll
+        for (int e = 0; e < 4; e++) ss = fmaf(v[e], v[e], ss);
     }
-    const float tot = pf_block_sum(ss, red);
+    const float tot = pf_block_sum<NW>(ss, red);
     const float rms = 1.0f / sqrtf(tot / (float)n + 1e-6f);
-    float4* xr = (float4*)(x + (size_t)t * n);
-    for (int i = threadIdx.x; i < n4; i += 256) {
-        const float4 v = tr[i], w4 = ((const float4*)w)[i];
-        float4 o = xr[i];
-        o.x = o.x + (v.x * rms) * (w4.x + 1.0f);
-        o.y = o.y + (v.y * rms) * (w4.y + 1.0f);
-        o.z = o.z + (v.z * rms) * (w4.z + 1.0f);
-        o.w = o.w + (v.w * rms) * (w4.w + 1.0f);
+    pf_f32x4* xr = (pf_f32x4*)(x + (size_t)t * n);
+    for (int i = threadIdx.x; i < n4; i += 64 * NW) {
+        const pf_f32x4 v = tr[i], w4 = ((const pf_f32x4*)w)[i];
+        pf_f32x4 o = xr[i];
+#pragma unroll
+        for (int e = 0; e < 4; e++) o[e] = o[e] + (v[e] * rms) * (w4[e] + 1.0f);
         xr[i] = o;
     }
 }
@@ -946,7 +978,9 @@ hipError_t launch_pf_postnorm_add(float* tmp, int T, int n, const float* w, floa
                                   const float* part, int nsp) {
     if (T <= 0) return hipSuccess;
     if (n % 4 != 0 || nsp < 0 || (nsp > 0 && part == nullptr)) return hipErrorInvalidValue;
-    k_pf_postnorm_add<<<T, 256, 0, st>>>(tmp, n, w, x, nsp > 0 ? part : tmp, nsp, (size_t)T * n);
+    const float* pt = nsp > 0 ? part : tmp;
+    if (T <= PF_FEW_ROWS) k_pf_postnorm_add<16><<<T, 1024, 0, st>>>(tmp, n, w, x, pt, nsp, (size_t)T * n);
+    else k_pf_postnorm_add<4><<<T, 256, 0, st>>>(tmp, n, w, x, pt, nsp, (size_t)T * n);
     return hipGetLastError();
 }
 
