@@ -14,9 +14,10 @@ struct PfKernel {
     int bm, bn, threads;
     double block_us;
 };
-// a launch's form: the tile type all its segments share, or segments of different tile types
-enum { PF_FORM_MIX = 1000 };
-// bm 64 or 128 (x 256 weight rows)
+// a launch's form: the type its tile-interleaved segments share, PF_FORM_MIX when they differ, or
+// PF_FORM_ROWS + the type of GGUF rows (rows of whole 256-element blocks)
+enum { PF_FORM_ROWS = 100, PF_FORM_MIX = 1000 };
+// bm 64 or 128 (x 256 weight rows); .k null for a form without one
 PfKernel pf_gemm8_kernel(int form, int bm);
 
 }  // namespace fllm

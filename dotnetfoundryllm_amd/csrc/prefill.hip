@@ -8,8 +8,9 @@
 // GEMM numerics: fp16 matrix cores (v_mfma_f32_16x16x32_f16, exact fp16 products summed in f32) on
 // operands of 22 significant bits. launch_pf_split scales each token row of X by a power of two so
 // that its largest magnitude lies in [2^14, 2^15) and writes hi = fp16(x) and lo = fp16(x - hi); the
-// epilogues undo the scale exactly. Tile-interleaved weights enter as exact integers (pf_gemm8.hip); GGUF
-// rows (pf_gemm_tile_h) dequantized exactly (the Dequantizer arithmetic), scaled by a per-matrix power of
+// epilogues undo the scale exactly. Tile-interleaved weights and rows of whole 256-element blocks
+// enter as they are stored, exact integers or halves (pf_gemm8.hip); the other GGUF rows
+// (pf_gemm_tile_h) dequantized exactly (the Dequantizer arithmetic), scaled by a per-matrix power of
 // two (pf_wexp) and split hi / lo; hi_x hi_w + hi_x lo_w + lo_x hi_w, within 2^-21 of the f32 product.
 #include "prefill.hpp"
 #include "deq.hpp"
@@ -731,7 +732,7 @@ hipError_t launch_pf_gemm(PfGemm a, int n_cu, hipStream_t st, int* pending) {
     if (a.nseg > 3 || a.K <= 0 || a.K % 32 != 0 || a.ldx < a.K || a.ldx % 4 != 0) return hipErrorInvalidValue;
     if (a.xh == nullptr || a.ldh < a.K || a.ldh % 8 != 0 || a.xs == nullptr) return hipErrorInvalidValue;
     const bool tiles = a.seg[0].layout == LAYOUT_TILES;
-    int form = tiles ? a.seg[0].type : -1;
+    int form = tiles ? a.seg[0].type : a.K % 256 == 0 ? PF_FORM_ROWS + a.seg[0].type : -1;
     for (int i = 0; i < a.nseg; i++) {
         const PfSeg& g = a.seg[i];
         if (g.N <= 0 || g.ldy < g.N || (g.layout == LAYOUT_TILES) != tiles) return hipErrorInvalidValue;
@@ -765,22 +766,23 @@ hipError_t launch_pf_gemm(PfGemm a, int n_cu, hipStream_t st, int* pending) {
     int nsplit = 1, nbk = 0;
     int64_t col_tiles = 0;
     double best = 0.0;
-    for (int c = 0; c < (tiles ? 2 : 1); c++) {
-        PfKernel kc = tiles ? pf_gemm8_kernel(form, c == 0 ? 64 : 128)
-                            : PfKernel{pf_rows_kernel_h<64>(a.seg[0].type), pf_gemm_lds_h<64>(), 64, PF_BN, 256, 0.0};
-        if (kc.k == nullptr) return hipErrorInvalidValue;
+    const bool big = pf_gemm8_kernel(form, 64).k != nullptr;
+    if (tiles && !big) return hipErrorInvalidValue;
+    for (int c = 0; c < (big ? 2 : 1); c++) {
+        const PfKernel kc = big ? pf_gemm8_kernel(form, c == 0 ? 64 : 128)
+                                : PfKernel{pf_rows_kernel_h<64>(a.seg[0].type), pf_gemm_lds_h<64>(), 64, PF_BN, 256, 0.0};
         hipError_t e = pf_lds_attr((const void*)kc.k, kc.lds);
         if (e != hipSuccess) return e;
         int64_t ct = 0;
         for (int i = 0; i < a.nseg; i++) ct += (a.seg[i].N + kc.bn - 1) / kc.bn;
         const int64_t base = ct * ((a.T + kc.bm - 1) / kc.bm);
-        const int per_cu = tiles ? 1 : pf_resident(kc);
+        const int per_cu = big ? 1 : pf_resident(kc);
         const int64_t slots = (int64_t)(per_cu > 0 ? per_cu : 1) * cus;
         // the row kernels: about 0.0118 us per resident slot and block
-        const double block_us = tiles ? kc.block_us : 0.0118 * (double)slots;
+        const double block_us = big ? kc.block_us : 0.0118 * (double)slots;
         // grids of three or more waves unsplit (there the last wave's share is small and the
         // reduction's cost was not repaid: Gemma-2-9B's o at 4096 tokens ran 6% longer in 2 parts)
-        const int nmax = side_by_side && per_cu > 0 && (base + slots - 1) / slots <= 2 ? (tiles ? 16 : 4) : 1;
+        const int nmax = side_by_side && per_cu > 0 && (base + slots - 1) / slots <= 2 ? (big ? 16 : 4) : 1;
         for (int n = 1; n == 1 || (n <= nmax && n <= nb); n++) {
             if (n > 1 && (size_t)(n - 1) * (size_t)a.T * (size_t)a.seg[0].ldy > a.part_cap) break;
             const int64_t waves = (base * n + slots - 1) / slots;
@@ -788,7 +790,7 @@ hipError_t launch_pf_gemm(PfGemm a, int n_cu, hipStream_t st, int* pending) {
             if (n > 1 && (n - 1) * bpp >= nb) continue;  // every part holds at least one block
             // a split has to win by 5% (at 4096 tokens, 14336 -> 3584 in 4 parts modelled 3% better and
             // ran even, its 235 MB of parts slowing the next kernel by 20 us)
-            const double cost = (double)waves * (bpp * block_us + (tiles ? PF_WAVE_US : 0.0)) +
+            const double cost = (double)waves * (bpp * block_us + (big ? PF_WAVE_US : 0.0)) +
                                 2 * (n - 1) * out_bytes / 4.0e6;
             if (k.k == nullptr || cost * (n > 1 ? 1.05 : 1.0) < best) {
                 best = cost;

@@ -287,22 +287,27 @@ def test_prefill_argument_contract(ctx):
         m.close()
 
 
-@pytest.mark.parametrize("types", [("q4_k",) * 7, ("q5_k",) * 7, ("q6_k",) * 7, ("q8_0",) * 7,
-                                   ("q5_k", "q8_0", "q6_k", "q4_k", "q4_k", "q6_k", "q5_k")],
-                         ids=["q4_k", "q5_k", "q6_k", "q8_0", "mixed"])
-def test_prefill_gemm_tile_edges(ctx, types):
-    """The tile-interleaved GEMMs at the edges of their tiles (64 and 128 tokens x 256 weight rows):
-    1 to 200 tokens on 128-, 512- and 768-row matrices of 2 and 3 blocks, every tile type alone and
-    launches that mix them. K / V rows of both layers (the second layer's carry every GEMM of the
-    first) against the oracle. Bound: operands of 22 bits or more and f32 sums of at most 768
-    products, 2^-22 + sqrt(768) 2^-24 (2e-6) for a projection, five of them in a row: 1e-5; twice that.
-    The softmax multiplies a score's relative error by the score, and these seeded weights make
-    scores q k of about 5e4 (|q|, |k| about 27 over 64 elements): Gemma-2's own attention scale, here
-    1e-5, keeps the scores below 1 and the bound that of the GEMMs. It is the median row's; a row whose
-    sums nearly cancel (the seeded weights are not zero-mean) has the file's bar."""
-    name_of = {"q4_k": N.Q4_K, "q5_k": N.Q5_K, "q6_k": N.Q6_K, "q8_0": N.Q8_0}
-    t = [name_of[x] for x in types]
-    cfg = dict(CONFIGS["test-gemma2"], n_layers=2, hidden=512, n_heads=8, n_kv_heads=2, head_dim=64, ffn=768, max_ctx=256,
+@pytest.mark.parametrize("types,hidden", [
+    ("q4_k", 512), ("q5_k", 512), ("q6_k", 512), ("q8_0", 512), ("q5_k q8_0 q6_k q4_k q4_k q6_k q5_k", 512),
+    ("q4_k", 2304), ("q5_k", 2304), ("q6_k", 2304), ("q8_0", 2304), ("q4_0", 512), ("f16", 512), ("q4_0", 352)],
+    ids=["q4_k", "q5_k", "q6_k", "q8_0", "mixed", "q4_k-rows", "q5_k-rows", "q6_k-rows", "q8_0-rows", "q4_0", "f16",
+         "q4_0-352"])
+def test_prefill_gemm_tile_edges(ctx, types, hidden):
+    """The large-tile GEMMs at the edges of their tiles (64 and 128 tokens x 256 weight rows): 2 to
+    200 tokens on 128-, 512- and 768-row matrices, every tile-interleaved type alone, launches that mix
+    them, and GGUF rows (2304 = 9 blocks has no tile layout, Q4_0 and F16 none at all; 352 is no whole
+    number of blocks and stays on the general row kernel). K / V rows of both layers (the second
+    layer's carry every GEMM of the first) against the oracle. Bound: operands of 22 bits or more and
+    f32 sums of at most 2304 products, 2^-22 + sqrt(2304) 2^-24 (3e-6) for a projection, five of them
+    in a row: 1.5e-5; a third more. The softmax multiplies a score's relative error by the score, and
+    these seeded weights make scores q k of about 5e4 (|q|, |k| about 27 over 64 elements): Gemma-2's
+    own attention scale, here 1e-5, keeps the scores below 1 and the bound that of the GEMMs. It is
+    the median row's; a row whose sums nearly cancel (the seeded weights are not zero-mean) has the
+    file's bar."""
+    name_of = {"q4_k": N.Q4_K, "q5_k": N.Q5_K, "q6_k": N.Q6_K, "q8_0": N.Q8_0, "q4_0": N.Q4_0, "f16": N.F16}
+    t = [name_of[x] for x in types.split()]
+    t = t * 7 if len(t) == 1 else t
+    cfg = dict(CONFIGS["test-gemma2"], n_layers=2, hidden=hidden, n_heads=8, n_kv_heads=2, head_dim=64, ffn=768, max_ctx=256,
                window=0x7FFFFFFF,
                types=dict(zip(("q", "k", "v", "o", "gate", "up", "down", "out"), t + [t[0]])))
     desc = desc_of(cfg)
