@@ -191,9 +191,15 @@ struct fllm_seq {
     float* hidden_dbg = nullptr;
     bool debug = false;
     bool use_graph = true;
-    bool graph_valid = false;
-    hipGraph_t graph = nullptr;
-    hipGraphExec_t gexec = nullptr;
+    // captured steps: of a Forward call; of the greedy loop (its last launch also starts the next step);
+    // of GREEDY_RUN steps of it
+    enum { G_FORWARD, G_GREEDY, G_RUN, G_COUNT };
+    struct StepGraph {
+        bool valid = false;
+        hipGraph_t graph = nullptr;
+        hipGraphExec_t exec = nullptr;
+    } graphs[G_COUNT];
+    int greedy_steps = 0;  // taken by the greedy loop, up to GREEDY_RUN_AFTER
     // profiling
     bool profile = false;
     std::vector<hipEvent_t> ev;
@@ -846,8 +852,10 @@ static hipError_t seq_alloc(fllm_seq* s, T** p, size_t count) {
 static void seq_free(fllm_seq* s) {
     if (s->pin) hipHostFree(s->pin);
     for (void* p : s->pf_allocs) hipFree(p);
-    if (s->gexec) hipGraphExecDestroy(s->gexec);
-    if (s->graph) hipGraphDestroy(s->graph);
+    for (auto& g : s->graphs) {
+        if (g.exec) hipGraphExecDestroy(g.exec);
+        if (g.graph) hipGraphDestroy(g.graph);
+    }
     for (void* p : s->allocs) hipFree(p);
     for (auto e : s->ev) hipEventDestroy(e);
     if (s->st) hipStreamDestroy(s->st);
@@ -1074,6 +1082,10 @@ extern "C" int32_t fllm_seq_set_graph(fllm_seq* s, int32_t enable) {
     return FLLM_OK;
 }
 
+static void invalidate_graphs(fllm_seq* s) {
+    for (auto& g : s->graphs) g.valid = false;
+}
+
 extern "C" int32_t fllm_seq_set_prefill_chunk(fllm_seq* s, int32_t tokens) {
     NOT_NULL(s);
     if (tokens < 1) return fail(FLLM_E_ARG_RANGE, "prefill chunk must be >= 1 token");
@@ -1083,7 +1095,7 @@ extern "C" int32_t fllm_seq_set_prefill_chunk(fllm_seq* s, int32_t tokens) {
 
 extern "C" int32_t fllm_seq_set_debug(fllm_seq* s, int32_t enable) {
     NOT_NULL(s);
-    if (s->debug != (enable != 0)) s->graph_valid = false;
+    if (s->debug != (enable != 0)) invalidate_graphs(s);
     s->debug = enable != 0;
     return FLLM_OK;
 }
@@ -1091,7 +1103,7 @@ extern "C" int32_t fllm_seq_set_debug(fllm_seq* s, int32_t enable) {
 extern "C" int32_t fllm_seq_set_attention_merge(fllm_seq* s, int32_t in_launch) {
     NOT_NULL(s);
     s->attn_merge_in = in_launch != 0;
-    s->graph_valid = false;  // the next graph replay captures the launches again
+    invalidate_graphs(s);  // the next graph replay captures the launches again
     return FLLM_OK;
 }
 
@@ -1244,8 +1256,41 @@ static hipError_t gemv_step(fllm_seq* s, const Tensor& t, const float* xf, float
     return hipSuccess;
 }
 
+static bool mfma_launch(const Tensor* const* t, int n, int glu, int64_t cols);
+
+// The start of a step that the launch fixing its token makes: the embedding row and the first
+// projection's table, when that projection runs on the matrix cores (it reads the table) and the row fits
+// the one workgroup that makes it.
+static bool step_embed(const fllm_seq* s, StepEmb* e) {
+    const fllm_model* m = s->m;
+    const fllm_model_desc& d = m->d;
+    if (!s->fused || d.hidden % 256 != 0 || d.hidden > STEP_EMB_MAX) return false;
+    const Layer& L = m->layers[0];
+    const Tensor* qkv[3] = {&L.q, &L.k, &L.v};
+    if (!mfma_launch(qkv, 3, 0, d.hidden)) return false;
+    e->emb = m->tok_embd.ptr; e->type = m->tok_embd.type; e->hidden = d.hidden; e->vocab = d.vocab;
+    e->w = L.attn_norm; e->norm_kind = d.arch == FLLM_ARCH_GEMMA2 ? 1 : 0;
+    e->x = s->x; e->tab = s->tab_x; e->ssq = s->ssq_x;
+    return true;
+}
+
+static hipError_t step_params(fllm_seq* s, int token, int pos) {
+    StepEmb e;
+    return step_embed(s, &e) ? launch_set_params_embed(s->params, token, pos, s->cur_len, e, s->st)
+                             : launch_set_params(s->params, token, pos, s->cur_len, s->st);
+}
+
+// the greedy token of the head's n keys, and the advance to the next step; start_next: with that step's
+// start (the greedy loop: a Forward call's token is the caller's, and step_params starts its step)
+static hipError_t step_advance(fllm_seq* s, int n, bool start_next) {
+    StepEmb e;
+    STEP("argmax", 8.0 * n, start_next && step_embed(s, &e) ? launch_argmax_keys_embed(s->head_keys, n, s->params, s->tokens_out, s->max_seq, e, s->st)
+                                              : launch_argmax_keys(s->head_keys, n, s->params, s->tokens_out, s->max_seq, s->st));
+    return hipSuccess;
+}
+
 // LM head, logits softcap, greedy argmax and the step advance (generic kernels).
-static hipError_t head_generic(fllm_seq* s) {
+static hipError_t head_generic(fllm_seq* s, bool start_next) {
     fllm_model* m = s->m;
     const fllm_model_desc& d = m->d;
     bool gemma = d.arch == FLLM_ARCH_GEMMA2;
@@ -1258,9 +1303,7 @@ static hipError_t head_generic(fllm_seq* s) {
     if (gemma && d.final_softcap > 0.0f) STEP("softcap", 8.0 * d.vocab, launch_softcap(s->logits, d.vocab, d.final_softcap, s->st));
     // (one kernel per profiled step: the segment keys, then their reduction and the step advance)
     STEP("argmax_segments", 4.0 * d.vocab, launch_argmax_seg(s->logits, d.vocab, s->head_keys, s->st));
-    STEP("argmax", 8.0 * argmax_segments(d.vocab),
-         launch_argmax_keys(s->head_keys, argmax_segments(d.vocab), s->params, s->tokens_out, s->max_seq, s->st));
-    return hipSuccess;
+    return step_advance(s, argmax_segments(d.vocab), start_next);
 }
 
 // true when a launch over these matrices (GLU: gate, up) runs the matrix-core variant
@@ -1281,7 +1324,7 @@ static bool mfma_launch(const Tensor* const* t, int n, int glu, int64_t cols) {
 // residual epilogues (Wo, down) write the table of x times the next RMSNorm weight plus partial
 // sums of squares, the gate/up epilogue the table of the FFN activation, and the next launch
 // copies it instead of quantizing the vector in every workgroup.
-static hipError_t enqueue_body_fused(fllm_seq* s) {
+static hipError_t enqueue_body_fused(fllm_seq* s, bool start_next) {
     fllm_model* m = s->m;
     const fllm_model_desc& d = m->d;
     bool gemma = d.arch == FLLM_ARCH_GEMMA2;
@@ -1289,14 +1332,17 @@ static hipError_t enqueue_body_fused(fllm_seq* s) {
     float eps = gemma ? 1e-6f : d.norm_eps;
     int nk = gemma ? 1 : 0;
     size_t layer_kv = (size_t)s->max_seq * kvdim;
-    // F32 / F16 / BF16 embedding rows are read by the first projection's prologue; quantized
-    // ones go through the element-wise lookup kernel first
+    // the step's embedding row and first table come with its parameters (step_embed); else F32 / F16 /
+    // BF16 rows are read by the first projection's prologue, and quantized ones go through the
+    // element-wise lookup kernel first
+    StepEmb se;
+    const bool emb_tab = step_embed(s, &se);
     int et = m->tok_embd.type;
-    bool emb_fused = et == FLLM_TYPE_F32 || et == FLLM_TYPE_F16 || et == FLLM_TYPE_BF16;
-    if (!emb_fused) STEP("embed", 4.0 * H, launch_embed(m->tok_embd.ptr, et, H, s->params, s->x, s->st));
+    bool emb_fused = !emb_tab && (et == FLLM_TYPE_F32 || et == FLLM_TYPE_F16 || et == FLLM_TYPE_BF16);
+    if (!emb_tab && !emb_fused) STEP("embed", 4.0 * H, launch_embed(m->tok_embd.ptr, et, H, s->params, s->x, s->st));
     const Tensor* head_t[1] = {&m->output};
     const bool head_mf = s->head_fused && !s->debug && mfma_launch(head_t, 1, 0, H);
-    bool xtab = false;  // tab_x / ssq_x hold the table of the current x for the next launch's norm
+    bool xtab = emb_tab;  // tab_x / ssq_x hold the table of the current x for the next launch's norm
     // Gemma-2 post-norms (x += GemmaRmsNorm(tmp, w) after o and after down): the pending one (its
     // weight pend) is folded into the prologue of the next launch that normalizes x on the matrix
     // cores (XIN_POST), which stores the new residual in the other of two buffers; cur is the
@@ -1410,7 +1456,7 @@ static hipError_t enqueue_body_fused(fllm_seq* s) {
         pend = nullptr;
         cur = s->x;
     }
-    if (!s->head_fused || s->debug) return head_generic(s);
+    if (!s->head_fused || s->debug) return head_generic(s, start_next);
     GemvArgs a{};
     a.nseg = 1;
     a.seg[0] = seg_of(m->output, EPI_LOGITS, s->logits, nullptr, nullptr);
@@ -1423,12 +1469,11 @@ static hipError_t enqueue_body_fused(fllm_seq* s) {
     size_t lds;
     int grid = gemv_plan(a, H, m->ctx->n_cu > 0 ? m->ctx->n_cu : 256, 0, &threads, &lds);
     STEP("lm_head", (double)m->output.bytes + 4.0 * (2.0 * H + d.vocab), launch_gemv_fused(a, grid, threads, lds, s->st));
-    STEP("argmax", 8.0 * grid, launch_argmax_keys(s->head_keys, grid, s->params, s->tokens_out, s->max_seq, s->st));
-    return hipSuccess;
+    return step_advance(s, grid, start_next);
 }
 
 // The decode step as one kernel per reference op (any tensor type and shape).
-static hipError_t enqueue_body_generic(fllm_seq* s) {
+static hipError_t enqueue_body_generic(fllm_seq* s, bool start_next) {
     fllm_model* m = s->m;
     const fllm_model_desc& d = m->d;
     bool gemma = d.arch == FLLM_ARCH_GEMMA2;
@@ -1468,35 +1513,47 @@ static hipError_t enqueue_body_generic(fllm_seq* s) {
         }
         if (s->debug) STEP("debug_copy", 8.0 * H, launch_copy_hidden(s->x, H, s->hidden_dbg + (size_t)l * H, s->st));
     }
-    return head_generic(s);
+    return head_generic(s, start_next);
 }
 
-static hipError_t enqueue_body(fllm_seq* s) { return s->fused ? enqueue_body_fused(s) : enqueue_body_generic(s); }
+static hipError_t enqueue_body(fllm_seq* s, bool start_next) {
+    return s->fused ? enqueue_body_fused(s, start_next) : enqueue_body_generic(s, start_next);
+}
+
+// Steps of the greedy loop captured together: about 8 us pass between two graph launches (Llama 4096
+// wide, two layers: 107 us of kernels in a step of 115), paid once per run. A run's graph costs about 100
+// us to make, the gain of four runs: it is made once a sequence has taken that many steps one by one.
+constexpr int GREEDY_RUN = 4, GREEDY_RUN_AFTER = 16;
+
+// replay of captured steps (captured first when they are not); the parameters are set
+static int32_t replay_step(fllm_seq* s, int kind) {
+    fllm_seq::StepGraph& g = s->graphs[kind];
+    if (!g.valid) {
+        if (g.exec) { hipGraphExecDestroy(g.exec); g.exec = nullptr; }
+        if (g.graph) { hipGraphDestroy(g.graph); g.graph = nullptr; }
+        HIP_TRY(hipStreamBeginCapture(s->st, hipStreamCaptureModeThreadLocal));
+        hipError_t e = hipSuccess;
+        const int n = kind == fllm_seq::G_RUN ? GREEDY_RUN : 1;
+        for (int i = 0; i < n && e == hipSuccess; i++) e = enqueue_body(s, kind != fllm_seq::G_FORWARD);
+        hipGraph_t cap = nullptr;
+        hipError_t e2 = hipStreamEndCapture(s->st, &cap);
+        if (e != hipSuccess) { if (cap) hipGraphDestroy(cap); return fail(FLLM_E_DEVICE, "capture: %s", hipGetErrorString(e)); }
+        if (e2 != hipSuccess) return fail(FLLM_E_DEVICE, "hipStreamEndCapture: %s", hipGetErrorString(e2));
+        g.graph = cap;
+        HIP_TRY(hipGraphInstantiate(&g.exec, g.graph, nullptr, nullptr, 0));
+        g.valid = true;
+    }
+    HIP_TRY(hipGraphLaunch(g.exec, s->st));
+    return FLLM_OK;
+}
 
 static int32_t enqueue_step(fllm_seq* s, int token, int pos) {
-    if (token >= 0) HIP_TRY(launch_set_params(s->params, token, pos, s->cur_len, s->st));
-    bool graph = s->use_graph && !s->profile;
-    if (!graph) {
-        hipError_t e = enqueue_body(s);
-        if (e != hipSuccess) return fail(FLLM_E_DEVICE, "decode step: %s", hipGetErrorString(e));
-        e = prof_collect(s);
-        if (e != hipSuccess) return fail(FLLM_E_DEVICE, "profile: %s", hipGetErrorString(e));
-        return FLLM_OK;
-    }
-    if (!s->graph_valid) {
-        if (s->gexec) { hipGraphExecDestroy(s->gexec); s->gexec = nullptr; }
-        if (s->graph) { hipGraphDestroy(s->graph); s->graph = nullptr; }
-        HIP_TRY(hipStreamBeginCapture(s->st, hipStreamCaptureModeThreadLocal));
-        hipError_t e = enqueue_body(s);
-        hipGraph_t g = nullptr;
-        hipError_t e2 = hipStreamEndCapture(s->st, &g);
-        if (e != hipSuccess) { if (g) hipGraphDestroy(g); return fail(FLLM_E_DEVICE, "capture: %s", hipGetErrorString(e)); }
-        if (e2 != hipSuccess) return fail(FLLM_E_DEVICE, "hipStreamEndCapture: %s", hipGetErrorString(e2));
-        s->graph = g;
-        HIP_TRY(hipGraphInstantiate(&s->gexec, s->graph, nullptr, nullptr, 0));
-        s->graph_valid = true;
-    }
-    HIP_TRY(hipGraphLaunch(s->gexec, s->st));
+    HIP_TRY(step_params(s, token, pos));
+    if (s->use_graph && !s->profile) return replay_step(s, fllm_seq::G_FORWARD);
+    hipError_t e = enqueue_body(s, false);
+    if (e != hipSuccess) return fail(FLLM_E_DEVICE, "decode step: %s", hipGetErrorString(e));
+    e = prof_collect(s);
+    if (e != hipSuccess) return fail(FLLM_E_DEVICE, "profile: %s", hipGetErrorString(e));
     return FLLM_OK;
 }
 
@@ -1562,24 +1619,21 @@ extern "C" int32_t fllm_decode_greedy(fllm_seq* s, int32_t token, int32_t positi
     if (s->profile) return fail(FLLM_E_INVALID_OP, "the device-side decode loop does not run in profile mode");
     HIP_TRY(hipSetDevice(s->m->ctx->device));
     // parameters once; every replayed step then feeds its greedy token to the next on the device
-    HIP_TRY(launch_set_params(s->params, token, position, s->cur_len, s->st));
-    for (int i = 0; i < n_steps; i++) {
-        int32_t rc;
+    HIP_TRY(step_params(s, token, position));
+    for (int i = 0; i < n_steps;) {
+        const bool run = s->use_graph && s->greedy_steps >= GREEDY_RUN_AFTER && n_steps - i >= GREEDY_RUN;
+        int32_t rc = FLLM_OK;
         if (s->use_graph) {
-            rc = FLLM_OK;
-            if (!s->graph_valid) {
-                // capture without touching the parameters the first step already holds
-                rc = enqueue_step(s, -1, -1);
-            } else {
-                hipError_t e = hipGraphLaunch(s->gexec, s->st);
-                if (e != hipSuccess) rc = fail(FLLM_E_DEVICE, "hipGraphLaunch: %s", hipGetErrorString(e));
-            }
+            rc = replay_step(s, run ? fllm_seq::G_RUN : fllm_seq::G_GREEDY);
         } else {
-            hipError_t e = enqueue_body(s);
-            rc = e == hipSuccess ? FLLM_OK : fail(FLLM_E_DEVICE, "decode step: %s", hipGetErrorString(e));
+            hipError_t e = enqueue_body(s, true);
+            if (e != hipSuccess) rc = fail(FLLM_E_DEVICE, "decode step: %s", hipGetErrorString(e));
         }
         if (rc) return rc;
-        s->cur_len++;
+        const int done = run ? GREEDY_RUN : 1;
+        s->cur_len += done;
+        s->greedy_steps = std::min(s->greedy_steps + done, GREEDY_RUN_AFTER);
+        i += done;
     }
     HIP_TRY(hipMemcpyAsync(out_tokens, s->tokens_out, sizeof(int32_t) * (size_t)n_steps, hipMemcpyDeviceToHost, s->st));
     HIP_TRY(hipStreamSynchronize(s->st));
@@ -1877,7 +1931,7 @@ extern "C" int32_t fllm_prefill(fllm_seq* s, const int32_t* tokens, int32_t n, i
     e = hipMemcpyAsync(s->x, s->pf_x + (size_t)(T_last - 1) * d.hidden, sizeof(float) * (size_t)d.hidden,
                        hipMemcpyDeviceToDevice, s->st);
     if (e == hipSuccess) e = launch_set_params(s->params, tokens[n - 1], pos0 + n - 1, pos0 + n - 1, s->st);
-    if (e == hipSuccess) e = head_generic(s);
+    if (e == hipSuccess) e = head_generic(s, false);
     if (e == hipSuccess) e = prof_collect(s);
     if (e != hipSuccess) return fail(FLLM_E_DEVICE, "prefill head: %s", hipGetErrorString(e));
     s->argmax_valid = true;

@@ -6,6 +6,7 @@
 #include "kernels.hpp"
 
 #include "deq.hpp"
+#include "actab.hpp"
 #include "gemv.hpp"
 
 #include <math.h>
@@ -543,6 +544,117 @@ __global__ __launch_bounds__(256) void k_argmax_keys(const unsigned long long* _
 hipError_t launch_argmax_keys(const unsigned long long* keys, int n, StepParams* p, int* tokens_out, int tokens_cap,
                               hipStream_t st) {
     k_argmax_keys<<<1, 256, 0, st>>>(keys, n, p, tokens_out, tokens_cap);
+    return hipGetLastError();
+}
+
+// The step parameters of a call (KEYS: the greedy advance of k_argmax_keys) and the start of the step they
+// belong to (StepEmb). One workgroup, bound by latency: two dependent memory round trips (the token's keys,
+// then its row; the norm weights are loaded beside the keys). The first projection of a step had read
+// the embedding row and built the table in each of its workgroups, 9.0 us more than from a table
+// (Llama 4096 wide: 15.8 and 6.9 us); this launch takes 5.5 us where k_argmax_keys took 4.0.
+template <bool KEYS>
+__global__ __launch_bounds__(1024) void k_step_begin(const unsigned long long* __restrict__ keys, int n, StepParams* p,
+                                                     int* tokens_out, int tokens_cap, int token, int pos, int cur_len,
+                                                     const StepEmb e) {
+    __shared__ unsigned long long sk[16];
+    __shared__ float sx[STEP_EMB_MAX / 16 * 17];  // 17 floats per 16 elements: the halves' reads spread over the banks
+    const int tid = threadIdx.x;
+    constexpr int NP = STEP_EMB_MAX / 1024;
+    float w[NP];
+#pragma unroll
+    for (int j = 0; j < NP; j++) {
+        const int i = tid + 1024 * j;
+        w[j] = i < e.hidden ? e.w[i] : 0.0f;
+    }
+    if constexpr (KEYS) {
+        unsigned long long best = 0ull;
+        for (int i = tid; i < n; i += 1024) best = keys[i] > best ? keys[i] : best;
+        for (int o = 32; o > 0; o >>= 1) {
+            const unsigned long long ot = __shfl_xor(best, o);
+            best = ot > best ? ot : best;
+        }
+        if ((tid & 63) == 0) sk[tid >> 6] = best;
+        __syncthreads();
+        best = sk[0];
+#pragma unroll
+        for (int i = 1; i < 16; i++) best = sk[i] > best ? sk[i] : best;
+        token = (int)(0xFFFFFFFFu - (uint32_t)(best & 0xFFFFFFFFull));
+        if (tid == 0) {
+            p->argmax = token;
+            if (p->nstep >= 0 && p->nstep < tokens_cap) tokens_out[p->nstep] = token;
+            p->nstep = p->nstep + 1;
+            p->token = token;
+            p->pos = p->pos + 1;
+            p->cur_len = p->cur_len + 1;
+        }
+        if (token < 0 || token >= e.vocab) token = 0;  // no key (an empty vocabulary): any row, not used
+    } else if (tid == 0) {
+        p->token = token;
+        p->pos = pos;
+        p->cur_len = cur_len;
+        p->argmax = -1;
+        p->nstep = 0;
+    }
+    float v[NP];
+#pragma unroll
+    for (int j = 0; j < NP; j++) {
+        const int i = tid + 1024 * j;
+        v[j] = i < e.hidden ? deq_elem(e.type, e.emb, (int64_t)token * e.hidden + i) : 0.0f;
+    }
+#pragma unroll
+    for (int j = 0; j < NP; j++) {
+        const int i = tid + 1024 * j;
+        if (i >= e.hidden) continue;
+        e.x[i] = v[j];
+        float sq = v[j] * v[j];  // of the 16 lanes of a half
+#pragma unroll
+        for (int o = 1; o < 16; o <<= 1) sq += __shfl_xor(sq, o);
+        if ((i & 15) == 0) e.ssq[i >> 4] = sq;
+        sx[(i >> 4) * 17 + (i & 15)] = v[j] * (e.norm_kind ? 1.0f + w[j] : w[j]);
+    }
+    __syncthreads();
+    if (tid >= e.hidden / 16) return;
+    const int h16 = tid, g32 = h16 >> 1, half = h16 & 1, b = g32 >> 3, gg = g32 & 7;
+    float t[16], amax = 0.0f, sum = 0.0f;
+#pragma unroll
+    for (int i = 0; i < 16; i++) {
+        t[i] = sx[h16 * 17 + i];
+        amax = fmaxf(amax, fabsf(t[i]));
+        sum += t[i];
+    }
+    float sc, inv;
+    half_scale(amax, sc, inv);
+    int X[16];
+#pragma unroll
+    for (int i = 0; i < 16; i++) X[i] = quant_x(t[i], inv);
+    uint4 d2, d1, d0;
+    uint32_t* q2 = (uint32_t*)&d2;
+    uint32_t* q1 = (uint32_t*)&d1;
+    uint32_t* q0 = (uint32_t*)&d0;
+#pragma unroll
+    for (int j = 0; j < 4; j++) digits3_pack4(X[j], X[4 + j], X[8 + j], X[12 + j], q2[j], q1[j], q0[j]);
+    uint4* tab = (uint4*)e.tab;
+    const int s = 2 * (gg >> 2) + half, q = gg & 3;
+    tab[atab_index(b, s, q, 0)] = d2;
+    tab[atab_index(b, s, q, 1)] = d1;
+    tab[atab_index(b, s, q, 2)] = d0;
+    float* st = (float*)(tab + (size_t)(e.hidden / 256) * 48) + 4 * (8 * b + gg);
+    st[half] = sc;
+    st[2 + half] = sum;
+}
+
+static bool step_emb_ok(const StepEmb& e) { return e.hidden > 0 && e.hidden % 256 == 0 && e.hidden <= STEP_EMB_MAX; }
+
+hipError_t launch_set_params_embed(StepParams* p, int token, int pos, int cur_len, const StepEmb& e, hipStream_t st) {
+    if (!step_emb_ok(e)) return hipErrorInvalidValue;
+    k_step_begin<false><<<1, 1024, 0, st>>>(nullptr, 0, p, nullptr, 0, token, pos, cur_len, e);
+    return hipGetLastError();
+}
+
+hipError_t launch_argmax_keys_embed(const unsigned long long* keys, int n, StepParams* p, int* tokens_out, int tokens_cap,
+                                    const StepEmb& e, hipStream_t st) {
+    if (!step_emb_ok(e)) return hipErrorInvalidValue;
+    k_step_begin<true><<<1, 1024, 0, st>>>(keys, n, p, tokens_out, tokens_cap, 0, 0, 0, e);
     return hipGetLastError();
 }
 

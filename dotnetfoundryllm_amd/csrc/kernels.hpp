@@ -35,6 +35,23 @@ hipError_t launch_gemv_tiles(const WMat& m, const float* xf, float* y, int n_cu,
 hipError_t launch_set_params(StepParams* p, int token, int pos, int cur_len, hipStream_t st);
 hipError_t launch_embed(const uint8_t* emb, int type, int hidden, const StepParams* p, float* x,
                         hipStream_t st);
+// The start of a step, made by the launch that fixes its token (set_params of a call, the greedy step
+// advance): x = E[token], and the first projection's activation table of x times its RMSNorm weight
+// (norm_kind 1: 1 + w) with the sums of squares of x per 16 elements. hidden: a multiple of 256, at
+// most STEP_EMB_MAX.
+constexpr int STEP_EMB_MAX = 8192;
+struct StepEmb {
+    const uint8_t* emb;
+    int type, hidden, vocab;
+    const float* w;
+    int norm_kind;
+    float* x;
+    void* tab;
+    float* ssq;
+};
+hipError_t launch_set_params_embed(StepParams* p, int token, int pos, int cur_len, const StepEmb& e, hipStream_t st);
+hipError_t launch_argmax_keys_embed(const unsigned long long* keys, int n, StepParams* p, int* tokens_out, int tokens_cap,
+                                    const StepEmb& e, hipStream_t st);
 // norm_kind 0: (x*rms)*w with eps; 1: Gemma (x*rms)*(1+w), eps 1e-6.
 hipError_t launch_rmsnorm(const float* x, const float* w, int n, float eps, int norm_kind, float* xn, hipStream_t st);
 hipError_t launch_qkv_post(float* q, float* k, float* v, const float* bq, const float* bk, const float* bv,

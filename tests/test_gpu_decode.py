@@ -502,3 +502,39 @@ def test_long_context_many_chunks(ctx, arch):
         orc.close()
         kv.close()
         m.close()
+
+@pytest.mark.parametrize("name", ["test-llama", "test-qwen2", "test-gemma2", "test-mixed"])
+def test_greedy_runs_and_single_steps_agree(ctx, name):
+    """The greedy loop in one call, in calls of every length up to 9 (single captured steps, then runs of
+    four with a remainder) and with Forward calls between them gives the tokens and the bits of the
+    logits of Forward calls alone: a step is the same launches, whoever fixes its token."""
+    cfg, desc, tensors = synthetic(name)
+    m = F.Model(ctx, desc)
+    upload(m, tensors)
+    n = min(50, desc.max_ctx - 2)
+    kv_a, kv_b = F.HipKvCache(m), F.HipKvCache(m)
+    fa, fb = F.HipForwardPass(m), F.HipForwardPass(m)
+    try:
+        tok, want = 3, []
+        for pos in range(n):
+            fa.forward(tok, pos, kv_a)
+            tok = fa.sample_greedy()
+            want.append(int(tok))
+        tok, pos, got, k = 3, 0, [], 0
+        while pos < n:
+            k = k % 9 + 1
+            step = min(k, n - pos)
+            if step == 5:  # a Forward call in the middle
+                fb.forward(tok, pos, kv_b)
+                out = [int(fb.sample_greedy())]
+            else:
+                out = [int(t) for t in fb.decode_greedy(tok, pos, step, kv_b)]
+            got += out
+            pos += len(out)
+            tok = got[-1]
+        assert got == want
+        assert np.array_equal(np.asarray(fa.logits), np.asarray(fb.logits))
+    finally:
+        kv_a.close()
+        kv_b.close()
+        m.close()
