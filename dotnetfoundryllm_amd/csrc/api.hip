@@ -1289,6 +1289,22 @@ static hipError_t step_advance(fllm_seq* s, int n, bool start_next) {
     return hipSuccess;
 }
 
+// true when the float projections of a normalized vector take these matrices in one launch
+static bool norm_gemv_launch(const Tensor* const* t, int n) {
+    for (int i = 0; i < n; i++)
+        if (t[i]->layout != LAYOUT_ROWS || t[i]->type != t[0]->type || t[i]->cols != t[0]->cols) return false;
+    return norm_gemv_ok(t[0]->type, t[0]->cols);
+}
+static NormGemv norm_gemv_args(const fllm_seq* s, const Tensor* const* t, int n, const float* norm_w) {
+    const fllm_model_desc& d = s->m->d;
+    const bool gemma = d.arch == FLLM_ARCH_GEMMA2;
+    NormGemv a{};
+    a.type = t[0]->type; a.cols = t[0]->cols; a.x = s->x; a.norm_w = norm_w;
+    a.eps = gemma ? 1e-6f : d.norm_eps; a.norm_kind = gemma ? 1 : 0; a.act = gemma ? 1 : 0;
+    for (int i = 0; i < n; i++) { a.w[i] = t[i]->ptr; a.rows[i] = (int)t[i]->rows; }
+    return a;
+}
+
 // LM head, logits softcap, greedy argmax and the step advance (generic kernels).
 static hipError_t head_generic(fllm_seq* s, bool start_next) {
     fllm_model* m = s->m;
@@ -1296,10 +1312,17 @@ static hipError_t head_generic(fllm_seq* s, bool start_next) {
     bool gemma = d.arch == FLLM_ARCH_GEMMA2;
     float eps = gemma ? 1e-6f : d.norm_eps;
     int H = d.hidden;
-    STEP("rmsnorm", 12.0 * H, launch_rmsnorm(s->x, m->out_norm, H, eps, gemma ? 1 : 0, s->xn, s->st));
-    if (s->debug) STEP("debug_copy", 8.0 * H, launch_copy_hidden(s->xn, H, s->hidden_dbg + (size_t)d.n_layers * H, s->st));
-    hipError_t e = gemv_step(s, m->output, s->xn, s->logits, nullptr);
-    if (e != hipSuccess) return e;
+    const Tensor* head_t[1] = {&m->output};
+    if (!s->debug && norm_gemv_launch(head_t, 1)) {
+        NormGemv a = norm_gemv_args(s, head_t, 1, m->out_norm);
+        a.out = s->logits;
+        STEP("norm_lm_head", (double)m->output.bytes + 4.0 * (2.0 * H + d.vocab), launch_norm_gemv(a, s->st));
+    } else {
+        STEP("rmsnorm", 12.0 * H, launch_rmsnorm(s->x, m->out_norm, H, eps, gemma ? 1 : 0, s->xn, s->st));
+        if (s->debug) STEP("debug_copy", 8.0 * H, launch_copy_hidden(s->xn, H, s->hidden_dbg + (size_t)d.n_layers * H, s->st));
+        hipError_t e = gemv_step(s, m->output, s->xn, s->logits, nullptr);
+        if (e != hipSuccess) return e;
+    }
     if (gemma && d.final_softcap > 0.0f) STEP("softcap", 8.0 * d.vocab, launch_softcap(s->logits, d.vocab, d.final_softcap, s->st));
     // (one kernel per profiled step: the segment keys, then their reduction and the step advance)
     STEP("argmax_segments", 4.0 * d.vocab, launch_argmax_seg(s->logits, d.vocab, s->head_keys, s->st));
@@ -1484,16 +1507,27 @@ static hipError_t enqueue_body_generic(fllm_seq* s, bool start_next) {
     STEP("embed", 4.0 * H, launch_embed(m->tok_embd.ptr, m->tok_embd.type, H, s->params, s->x, s->st));
     for (int l = 0; l < d.n_layers; l++) {
         const Layer& L = m->layers[(size_t)l];
-        STEP("rmsnorm", 12.0 * H, launch_rmsnorm(s->x, L.attn_norm, H, eps, nk, s->xn, s->st));
-        hipError_t e;
-        if ((e = gemv_step(s, L.q, s->xn, s->q, nullptr)) != hipSuccess) return e;
-        if ((e = gemv_step(s, L.k, s->xn, s->k, nullptr)) != hipSuccess) return e;
-        if ((e = gemv_step(s, L.v, s->xn, s->v, nullptr)) != hipSuccess) return e;
         float* kc = s->kc + (size_t)l * layer_kv;
         float* vc = s->vc + (size_t)l * layer_kv;
-        STEP("qkv_rope_kvstore", 8.0 * (m->qdim + 2 * kvdim),
-             launch_qkv_post(s->q, s->k, s->v, L.bq, L.bk, L.bv, s->rope, d.n_heads, d.n_kv_heads, d.head_dim, kc, vc,
-                             s->params, s->st));
+        hipError_t e;
+        const Tensor* qkv_t[3] = {&L.q, &L.k, &L.v};
+        const Tensor* gu_t[2] = {&L.gate, &L.up};
+        if (norm_gemv_launch(qkv_t, 3) && d.head_dim % 2 == 0) {
+            NormGemv a = norm_gemv_args(s, qkv_t, 3, L.attn_norm);
+            a.bias[0] = L.bq; a.bias[1] = L.bk; a.bias[2] = L.bv;
+            a.rope = s->rope; a.hd = d.head_dim; a.params = s->params;
+            a.out = s->q; a.kc = kc; a.vc = vc;
+            STEP("norm_qkv_rope_kv", (double)(L.q.bytes + L.k.bytes + L.v.bytes) + 4.0 * (2.0 * H + m->qdim + 2 * kvdim),
+                 launch_norm_gemv_qkv(a, s->st));
+        } else {
+            STEP("rmsnorm", 12.0 * H, launch_rmsnorm(s->x, L.attn_norm, H, eps, nk, s->xn, s->st));
+            if ((e = gemv_step(s, L.q, s->xn, s->q, nullptr)) != hipSuccess) return e;
+            if ((e = gemv_step(s, L.k, s->xn, s->k, nullptr)) != hipSuccess) return e;
+            if ((e = gemv_step(s, L.v, s->xn, s->v, nullptr)) != hipSuccess) return e;
+            STEP("qkv_rope_kvstore", 8.0 * (m->qdim + 2 * kvdim),
+                 launch_qkv_post(s->q, s->k, s->v, L.bq, L.bk, L.bv, s->rope, d.n_heads, d.n_kv_heads, d.head_dim, kc, vc,
+                                 s->params, s->st));
+        }
         if ((e = attention_step(s, l, kc, vc, false)) != hipSuccess) return e;
         if (gemma) {
             if ((e = gemv_step(s, L.o, s->att, s->tmp, nullptr)) != hipSuccess) return e;
@@ -1501,10 +1535,16 @@ static hipError_t enqueue_body_generic(fllm_seq* s, bool start_next) {
         } else {
             if ((e = gemv_step(s, L.o, s->att, s->x, s->x)) != hipSuccess) return e;
         }
-        STEP("rmsnorm", 12.0 * H, launch_rmsnorm(s->x, L.ffn_norm, H, eps, nk, s->xn, s->st));
-        if ((e = gemv_step(s, L.gate, s->xn, s->g, nullptr)) != hipSuccess) return e;
-        if ((e = gemv_step(s, L.up, s->xn, s->u, nullptr)) != hipSuccess) return e;
-        STEP("ffn_act", 12.0 * d.ffn, launch_act(s->g, s->u, d.ffn, gemma ? 1 : 0, s->h, s->st));
+        if (norm_gemv_launch(gu_t, 2)) {
+            NormGemv a = norm_gemv_args(s, gu_t, 2, L.ffn_norm);
+            a.out = s->h;
+            STEP("norm_gate_up_act", (double)(L.gate.bytes + L.up.bytes) + 4.0 * (2.0 * H + d.ffn), launch_norm_gemv_glu(a, s->st));
+        } else {
+            STEP("rmsnorm", 12.0 * H, launch_rmsnorm(s->x, L.ffn_norm, H, eps, nk, s->xn, s->st));
+            if ((e = gemv_step(s, L.gate, s->xn, s->g, nullptr)) != hipSuccess) return e;
+            if ((e = gemv_step(s, L.up, s->xn, s->u, nullptr)) != hipSuccess) return e;
+            STEP("ffn_act", 12.0 * d.ffn, launch_act(s->g, s->u, d.ffn, gemma ? 1 : 0, s->h, s->st));
+        }
         if (gemma) {
             if ((e = gemv_step(s, L.down, s->h, s->tmp, nullptr)) != hipSuccess) return e;
             STEP("postnorm_add", 12.0 * H, launch_postnorm_add(s->tmp, L.post_ffn, H, s->x, s->x, s->st));

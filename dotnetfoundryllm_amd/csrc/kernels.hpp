@@ -32,6 +32,32 @@ hipError_t launch_gemv(const WMat& m, const float* xf, float* y, const float* re
 // y = W x for a matrix in the tile-interleaved layout (launch_pack_tiles): matrix-core variant only
 hipError_t launch_gemv_tiles(const WMat& m, const float* xf, float* y, int n_cu, hipStream_t st);
 
+// Projections of RmsNorm(x) by F32 / F16 / BF16 matrices of one type, one launch for all of them
+// (cols a multiple of 4, 2-byte types 8): q, k, v with bias, RoPE and the K / V store (even row counts and
+// head_dim); h = act(gate) * up (act 0 SiLU, 1 GELU); or plain rows (y = W RmsNorm(x)).
+struct NormGemv {
+    int type;
+    int64_t cols;
+    const float* x;
+    const float* norm_w;
+    float eps;
+    int norm_kind;
+    const uint8_t* w[3];
+    int rows[3];           // rows[1] = rows[2]: k and v
+    const float* bias[3];  // q, k, v: optional
+    const float2* rope;
+    int hd;
+    const StepParams* params;
+    float* out;            // q, h or y
+    float* kc;             // this layer's caches [pos][rows[1]]
+    float* vc;
+    int act;
+};
+bool norm_gemv_ok(int type, int64_t cols);
+hipError_t launch_norm_gemv_qkv(const NormGemv& a, hipStream_t st);
+hipError_t launch_norm_gemv_glu(const NormGemv& a, hipStream_t st);
+hipError_t launch_norm_gemv(const NormGemv& a, hipStream_t st);
+
 hipError_t launch_set_params(StepParams* p, int token, int pos, int cur_len, hipStream_t st);
 hipError_t launch_embed(const uint8_t* emb, int type, int hidden, const StepParams* p, float* x,
                         hipStream_t st);

@@ -538,3 +538,33 @@ def test_greedy_runs_and_single_steps_agree(ctx, name):
         kv_a.close()
         kv_b.close()
         m.close()
+
+
+@pytest.mark.parametrize("tt", [N.F32, N.F16, N.BF16], ids=["f32", "f16", "bf16"])
+@pytest.mark.parametrize("arch,hidden,ffn", [("test-llama", 256, 264), ("test-qwen2", 264, 72), ("test-gemma2", 1032, 520)],
+                         ids=["llama-256", "qwen2-264", "gemma2-1032"])
+def test_float_projections_of_a_norm(ctx, tt, arch, hidden, ffn):
+    """A model of one float type: norm + q/k/v + bias + RoPE + K/V store, norm + gate/up + activation and
+    norm + LM head as one launch each, on rows of less than, one and a half and several 64-lane loads,
+    1 + w norms and an odd vocabulary. Bound: f32 sums of at most 1032 products, sqrt(1032) 2^-24 (2e-6)
+    per projection, ten in a row, the oracle's own error as large: 4e-5."""
+    cfg = dict(CONFIGS[arch], n_layers=2, hidden=hidden, n_heads=4, n_kv_heads=2, head_dim=64, ffn=ffn, vocab=511,
+               max_ctx=64, window=0x7FFFFFFF, tied=False, emb_type=tt,
+               types={k: tt for k in ("q", "k", "v", "o", "gate", "up", "down", "out")})
+    desc = desc_of(cfg)
+    tensors = {e[0]: (e, synth_bytes(cfg, e)) for e in tensor_plan(cfg)}
+    m = F.Model(ctx, desc)
+    upload(m, tensors)
+    kv, fwd, orc = F.HipKvCache(m), F.HipForwardPass(m), O.OracleModel(desc, tensors)
+    try:
+        for pos, t in enumerate(F.synth_tokens(cfg["seed"], 3, desc.vocab, 20)):
+            fwd.forward(int(t), pos, kv)
+            assert orc.forward(int(t), pos) == 0
+            assert O.normwise_rel_err(fwd.logits, orc.logits()) <= 4e-5, pos
+        for l in range(desc.n_layers):
+            assert O.normwise_rel_err(kv.get_keys(l), orc.kv(l, 0)) <= 4e-5
+            assert O.normwise_rel_err(kv.get_values(l), orc.kv(l, 1)) <= 4e-5
+    finally:
+        orc.close()
+        kv.close()
+        m.close()
