@@ -2085,6 +2085,100 @@ hipError_t launch_pack_tiles(int type, const uint8_t* src, uint8_t* dst, int64_t
     return hipGetLastError();
 }
 
+// ---- small matrices of rows that are no whole chunks ------------------------------------------------
+// One wave per row, one 32-element group per lane and pass, exact f32 products. For matrices of at most
+// 2^21 elements and rows of at most 2048: there the launch is bound by its chain of memory latencies, and
+// k_gemv_fused's (the vector's quantization, the rows staged through LDS, 8 rows to a wave) took 8.0 us for
+// Q4_K 512 x 1408 where this one, two loads deep, takes 4.9. Longer rows read x at a stride of
+// 128 bytes per lane too often; larger matrices are bound by bytes, which the staging reads coalesced.
+struct __attribute__((packed, aligned(2))) Sm16 { uint32_t v[4]; };
+struct __attribute__((packed, aligned(2))) Sm8 { uint32_t v[2]; };
+template <int T>
+__device__ __forceinline__ float sm_group(const uint8_t* __restrict__ w, int64_t e0, const float* x) {
+    if constexpr (T == FLLM_TYPE_Q4_K || T == FLLM_TYPE_Q5_K) {
+        const uint8_t* p = w + (e0 >> 8) * (T == FLLM_TYPE_Q4_K ? 144 : 176);
+        const int g = (int)((e0 & 255) >> 5), sh = 8 * (g & 3);
+        const uint4 h = *(const uint4*)p;
+        const uint4 q4 = *(const uint4*)(p + (T == FLLM_TYPE_Q4_K ? 16 : 48) + 16 * g);
+        uint32_t hb = 0u;
+        if constexpr (T == FLLM_TYPE_Q5_K) hb = *(const uint32_t*)(p + 16 + 4 * g);
+        const uint32_t y = h.y >> sh, z = h.z >> sh, w4 = h.w >> sh;
+        const uint32_t sc = g < 4 ? (y & 63u) : ((w4 & 15u) | ((y >> 2) & 0x30u));
+        const uint32_t mn = g < 4 ? (z & 63u) : (((w4 >> 4) & 15u) | ((z >> 2) & 0x30u));
+        const uint32_t q[4] = {q4.x, q4.y, q4.z, q4.w};
+        float s = 0.0f, t = 0.0f;
+#pragma unroll
+        for (int i = 0; i < 32; i++) {
+            uint32_t c = (q[i >> 3] >> (4 * (i & 7))) & 15u;
+            if constexpr (T == FLLM_TYPE_Q5_K) c |= ((hb >> i) & 1u) << 4;
+            s = fmaf((float)c, x[i], s);
+            t += x[i];
+        }
+        return half_exact(h.x & 0xFFFFu) * (float)sc * s - half_exact(h.x >> 16) * (float)mn * t;
+    } else if constexpr (T == FLLM_TYPE_Q6_K) {
+        const uint8_t* p = w + (e0 >> 8) * 210;
+        const int g = (int)((e0 & 255) >> 5);
+        const Sm16 q = *(const Sm16*)(p + 16 * g);
+        const Sm8 h = *(const Sm8*)(p + 128 + 8 * g);
+        float s0 = 0.0f, s1 = 0.0f;
+#pragma unroll
+        for (int i = 0; i < 32; i++) {
+            const uint32_t c = ((q.v[i >> 3] >> (4 * (i & 7))) & 15u) | (((h.v[i >> 4] >> (2 * (i & 15))) & 3u) << 4);
+            if (i < 16) s0 = fmaf((float)((int)c - 32), x[i], s0);
+            else s1 = fmaf((float)((int)c - 32), x[i], s1);
+        }
+        const float d = half_exact(*(const uint16_t*)(p + 208));
+        return d * ((float)*(const int8_t*)(p + 192 + 2 * g) * s0 + (float)*(const int8_t*)(p + 193 + 2 * g) * s1);
+    } else if constexpr (T == FLLM_TYPE_Q8_0) {
+        const uint8_t* p = w + (e0 >> 5) * 34;
+        const Sm16 a = *(const Sm16*)(p + 2), b = *(const Sm16*)(p + 18);
+        float s = 0.0f;
+#pragma unroll
+        for (int i = 0; i < 16; i++) {
+            s = fmaf((float)(int8_t)(a.v[i >> 2] >> (8 * (i & 3))), x[i], s);
+            s = fmaf((float)(int8_t)(b.v[i >> 2] >> (8 * (i & 3))), x[16 + i], s);
+        }
+        return half_exact(*(const uint16_t*)p) * s;
+    } else {
+        const uint8_t* p = w + (e0 >> 5) * 18;
+        const Sm16 a = *(const Sm16*)(p + 2);
+        float s = 0.0f;
+#pragma unroll
+        for (int i = 0; i < 16; i++) {
+            const uint32_t c = a.v[i >> 2] >> (8 * (i & 3));
+            s = fmaf((float)((int)(c & 15u) - 8), x[i], s);
+            s = fmaf((float)((int)((c >> 4) & 15u) - 8), x[16 + i], s);
+        }
+        return half_exact(*(const uint16_t*)p) * s;
+    }
+}
+
+template <int T>
+__global__ __launch_bounds__(256) void k_gemv_small(const uint8_t* __restrict__ w, int rows, int G, const float* __restrict__ x,
+                                                    float* out, const float* resid) {
+    const int row = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
+    if (row >= rows) return;
+    const float rs = resid ? resid[row] : 0.0f;
+    float acc = 0.0f;
+    for (int g = lane; g < G; g += 64) {
+        float xv[32];
+#pragma unroll
+        for (int i = 0; i < 8; i++) *(float4*)(xv + 4 * i) = ((const float4*)(x + 32 * g))[i];
+        acc += sm_group<T>(w, ((int64_t)row * G + g) * 32, xv);
+    }
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) acc += __shfl_xor(acc, o);
+    if (lane == 0) out[row] = resid ? rs + acc : acc;
+}
+
+// plain projections of an f32 vector at these sizes (the q/k/v, gated and table-writing launches keep theirs)
+static bool gemv_small(const GemvArgs& a) {
+    const GemvSeg& sg = a.seg[0];
+    return !a.mfma && a.nseg == 1 && !a.glu && a.xin == XIN_F32 && a.tab_out == nullptr &&
+           (sg.epi == EPI_STORE || sg.epi == EPI_RESID) && sg.layout == LAYOUT_ROWS && a.G <= 64 &&
+           (int64_t)sg.rows * a.G <= (1 << 16) && (((uintptr_t)a.x | (uintptr_t)sg.w) & 15) == 0;
+}
+
 hipError_t launch_gemv_fused(const GemvArgs& a, int grid, int block_threads, size_t lds, hipStream_t st) {
     if (grid <= 0) return hipSuccess;
     // the matrix-core prologue always reads its input: the table, or the vector (cols floats)
@@ -2107,6 +2201,20 @@ hipError_t launch_gemv_fused(const GemvArgs& a, int grid, int block_threads, siz
         const MfKernel k = mf_kernel(a, kc);
         if (k == nullptr) return hipErrorInvalidValue;
         k<<<grid, block_threads, lds, st>>>(a);
+    } else if (gemv_small(a)) {
+        const GemvSeg& sg = a.seg[0];
+        const float* resid = sg.epi == EPI_RESID ? sg.resid : nullptr;
+        const int wgs = (sg.rows + 3) / 4;
+        if (wgs <= 0) return hipSuccess;
+        auto run = [&](auto k) { k<<<wgs, 256, 0, st>>>(sg.w, sg.rows, a.G, a.x, sg.out, resid); };
+        switch (sg.type) {
+            case FLLM_TYPE_Q4_K: run(k_gemv_small<FLLM_TYPE_Q4_K>); break;
+            case FLLM_TYPE_Q5_K: run(k_gemv_small<FLLM_TYPE_Q5_K>); break;
+            case FLLM_TYPE_Q6_K: run(k_gemv_small<FLLM_TYPE_Q6_K>); break;
+            case FLLM_TYPE_Q8_0: run(k_gemv_small<FLLM_TYPE_Q8_0>); break;
+            case FLLM_TYPE_Q4_0: run(k_gemv_small<FLLM_TYPE_Q4_0>); break;
+            default: return hipErrorInvalidValue;
+        }
     } else if (block_threads <= 512)
         k_gemv_fused<false><<<grid, block_threads, lds, st>>>(a);
     else

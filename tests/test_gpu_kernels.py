@@ -194,3 +194,17 @@ def test_gemv_argument_checks(ctx):
     finally:
         for b in (wb, xb, yb):
             b.close()
+
+
+@pytest.mark.parametrize("t", [N.Q4_K, N.Q5_K, N.Q6_K, N.Q8_0, N.Q4_0])
+@pytest.mark.parametrize("rows,cols", [(64, 32), (8, 352), (9, 1408), (1024, 2048), (1032, 2048), (64, 2080)])
+def test_gemv_small_matrices(ctx, t, rows, cols):
+    """Rows of at most 64 groups in matrices of at most 2^16 groups take one wave per row: one group,
+    rows that start inside a block, the last wave of a workgroup past the rows, both sides of the two
+    limits (1024 x 64 and 1032 x 64 groups, 65 groups a row)."""
+    if (rows * cols) % N.BLOCK[t][1]:
+        pytest.skip("not a whole number of blocks")
+    y, ref = run_gemv(ctx, t, rows, cols)
+    # sums of at most 2080 f32 products: sqrt(2080) 2^-24 of the row's absolute sum, which the file's
+    # bound covers for these weights
+    assert O.normwise_rel_err(y, ref) <= 1e-5
