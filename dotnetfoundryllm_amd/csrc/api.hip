@@ -108,7 +108,7 @@ struct Tensor {
     int type = -1;
     int64_t rows = 0, cols = 0;
     uint64_t bytes = 0;
-    int wexp = 0;  // batched prefill: 2^-wexp brings the largest |w| into [2^14, 2^15) (pf_wexp)
+    int wexp = 0;  // batched prefill: 2^-wexp brings the largest magnitude of launch_pf_wmax into [2^14, 2^15)
     bool present() const { return ptr != nullptr; }
     WMat mat() const { return WMat{ptr, type, rows, cols}; }
 };
@@ -781,8 +781,8 @@ extern "C" int32_t fllm_model_finalize(fllm_model* m) {
     if (!m->output_tied && tiles_launch_ok(head, 1, 0)) to_pack.push_back(&m->output);
     HIP_TRY(hipSetDevice(m->ctx->device));
     {
-        // the largest |w| of every projection matrix, for the batched prefill's fp16 split (read in
-        // GGUF row layout, before the regrouping)
+        // the largest magnitude that the batched prefill's fp16 operands scale, of every projection
+        // matrix (read in GGUF row layout, before the regrouping)
         std::vector<Tensor*> mats;
         for (Layer& L : m->layers) {
             Tensor* ts[7] = {&L.q, &L.k, &L.v, &L.o, &L.gate, &L.up, &L.down};
@@ -792,7 +792,7 @@ extern "C" int32_t fllm_model_finalize(fllm_model* m) {
         hipError_t e = hipMalloc(&dmax, sizeof(unsigned) * mats.size());
         if (e == hipSuccess) e = hipMemsetAsync(dmax, 0, sizeof(unsigned) * mats.size(), m->ctx->stream);
         for (size_t i = 0; i < mats.size() && e == hipSuccess; i++)
-            e = launch_pf_wmax(mats[i]->type, mats[i]->ptr, mats[i]->rows * mats[i]->cols, dmax + i, m->ctx->stream);
+            e = launch_pf_wmax(mats[i]->type, mats[i]->ptr, mats[i]->rows, mats[i]->cols, dmax + i, m->ctx->stream);
         std::vector<unsigned> hmax(mats.size(), 0u);
         if (e == hipSuccess)
             e = hipMemcpyAsync(hmax.data(), dmax, sizeof(unsigned) * mats.size(), hipMemcpyDeviceToHost, m->ctx->stream);

@@ -7,7 +7,9 @@
 //    MFMAs (x lo, x hi). A 256-element block's sum is scaled by its d in f32. Its min term is one more
 //    MFMA whose K slice packs, per row, (v_g hi, v_g lo, v_g hi) for v_g = -dmin m_g against, per token,
 //    the group sums (X_g hi, X_g hi, X_g lo); the group sums are stored times 2^-6 (to stay in fp16's
-//    range) and v_g taken times 2^6.
+//    range) and v_g times 2^-wexp, which brings the matrix's largest into [2^14, 2^15) (launch_pf_wmax), so
+//    the sums are held times 2^-(wexp + 6), d and the epilogue taking the factor. (v_g times a fixed 2^6
+//    had left its two halves' range from dmin m = 2047 on.)
 //  - Q6_K: w = d (sc q), |sc q| <= 4096: hi = fp16(sc q) and lo = sc q - hi (0 or +-1) hold it exactly;
 //    x lo hi + x hi lo + x hi hi (the dropped x lo lo is below 2^-22 of a product), d per block.
 //  - Q8_0, Q4_0: the code (Q4_0: minus 8), exact; two MFMAs, each 32-element block's sum scaled by its d.
@@ -345,6 +347,7 @@ __device__ __forceinline__ void g8_tile(const PfGemm& a, const PfSeg& sg, int n0
     // row r0 + 128 i of a stage: the swizzle depends on r0 alone
     const int so = r0 * G8_BK + ((ch ^ ((r0 >> 2) & 2)) << 3);
     const float wsc = ldexpf(1.0f, -sg.wexp);
+    const float msc = MIN ? wsc * 0.015625f : 1.0f;  // what the sums of the block-scaled forms are held times
     const int fe = F16 ? g8_f16_exp(sg.wexp) : 0;
     const _Float16 fh0 = (_Float16)ldexpf(1.0f, fe < 15 ? fe : 15), fh1 = (_Float16)ldexpf(1.0f, fe < 15 ? 0 : fe - 15);
     const g8_h2 fs0 = {fh0, fh0}, fs1 = {fh1, fh1};
@@ -463,11 +466,11 @@ __device__ __forceinline__ void g8_tile(const PfGemm& a, const PfSeg& sg, int n0
                 for (int i = 0; i < WC; i++) {
                     const int row = r0 + 128 * i;
                     if constexpr (MIN) {
-                        if (ch == 0) sd[row] = sign * g8_half(blk_c[i].hdr.x & 0xFFFFu);
-                        // v_g = -dmin m_g (exact in f32) of groups 2 ch, 2 ch + 1, times 2^6, split
+                        if (ch == 0) sd[row] = (sign * msc) * g8_half(blk_c[i].hdr.x & 0xFFFFu);
+                        // v_g = -dmin m_g (exact in f32) of groups 2 ch, 2 ch + 1, times 2^-wexp, split
                         const float dm = g8_half(blk_c[i].hdr.x >> 16);
                         const uint32_t mn = g8_mins(blk_c[i].hdr, ch);
-                        const float v0 = -(dm * (float)(mn & 0xFFu)) * 64.0f, v1 = -(dm * (float)(mn >> 8)) * 64.0f;
+                        const float v0 = -(dm * (float)(mn & 0xFFu)) * wsc, v1 = -(dm * (float)(mn >> 8)) * wsc;
                         const g8_p2 h = __builtin_amdgcn_cvt_pkrtz(v0, v1);
                         const g8_p2 l = __builtin_amdgcn_cvt_pkrtz(v0 - (float)h[0], v1 - (float)h[1]);
                         uint32_t* dv = (uint32_t*)(swv + row * G8_LDV) + ch;
@@ -572,7 +575,7 @@ __device__ __forceinline__ void g8_tile(const PfGemm& a, const PfSeg& sg, int n0
 
     // D lane l: column l & 15, rows 4 (l >> 4) + e. The residual values are loaded together, from
     // clamped addresses, before the first store.
-    const float wun = F16 ? ldexpf(1.0f, -fe) : SC == G8_SC_STEP ? ldexpf(1.0f, sg.wexp) : 1.0f;
+    const float wun = F16 ? ldexpf(1.0f, -fe) : SC == G8_SC_STEP ? ldexpf(1.0f, sg.wexp) : MIN ? ldexpf(1.0f, sg.wexp + 6) : 1.0f;
     const bool add = a.add && blockIdx.z == 0;
     float* out = blockIdx.z == 0 ? sg.y
                                  : a.part + (size_t)(blockIdx.z - 1) * a.T * sg.ldy + (size_t)(sg.y - a.seg[0].y);

@@ -660,11 +660,40 @@ __global__ __launch_bounds__(256) void k_pf_wmax(int type, const uint8_t* __rest
     }
 }
 
-hipError_t launch_pf_wmax(int type, const uint8_t* w, int64_t n, unsigned* out, hipStream_t st) {
-    if (n <= 0) return hipSuccess;
+// largest |dmin m| of the groups of n Q4_K / Q5_K blocks of `bytes` bytes, as float bits
+__global__ __launch_bounds__(256) void k_pf_mmax(int bytes, const uint8_t* __restrict__ w, int64_t n, unsigned* out) {
+    __shared__ float red[4];
+    float m = 0.0f;
+    for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (int64_t)gridDim.x * 256) {
+        const uint8_t* p = w + i * bytes;
+        const float dmin = fabsf(half_exact(deq_ld_u16(p + 2)));
+        int top = 0;
+#pragma unroll
+        for (int g = 0; g < 8; g++) {
+            int sc, mn;
+            kscale_min(p + 4, g, sc, mn);
+            top = mn > top ? mn : top;
+        }
+        const float v = dmin * (float)top;
+        m = v > m ? v : m;  // a NaN is skipped
+    }
+    m = pf_wave_max(m);
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = m;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        m = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
+        if (m > 0.0f) atomicMax(out, __float_as_uint(m));
+    }
+}
+
+hipError_t launch_pf_wmax(int type, const uint8_t* w, int64_t rows, int64_t cols, unsigned* out, hipStream_t st) {
+    const bool whole = cols % 256 == 0, mins = whole && (type == FLLM_TYPE_Q4_K || type == FLLM_TYPE_Q5_K);
+    if (rows * cols <= 0 || (whole && type == FLLM_TYPE_Q6_K)) return hipSuccess;
+    const int64_t n = mins ? rows * cols / 256 : rows * cols;
     int64_t blocks = (n + 255) / 256;
     if (blocks > 4096) blocks = 4096;
-    k_pf_wmax<<<(unsigned)blocks, 256, 0, st>>>(type, w, n, out);
+    if (mins) k_pf_mmax<<<(unsigned)blocks, 256, 0, st>>>(type == FLLM_TYPE_Q4_K ? 144 : 176, w, n, out);
+    else k_pf_wmax<<<(unsigned)blocks, 256, 0, st>>>(type, w, n, out);
     return hipGetLastError();
 }
 

@@ -19,7 +19,8 @@ struct PfSeg {
     float* y;   // [T][ldy], column 0 = weight row 0
     int ldy;
     int tiles;  // set by launch_pf_gemm: 128-row column tiles of the segment
-    int wexp;   // fp16 matrix cores: the weights enter scaled by 2^-wexp (launch_pf_wmax gives it)
+    int wexp;   // fp16 matrix cores: the weights (Q4_K / Q5_K rows of whole blocks: the offsets dmin m) enter
+                // scaled by 2^-wexp (launch_pf_wmax gives it)
 };
 struct PfGemm {
     const float* x;
@@ -66,10 +67,11 @@ hipError_t launch_pf_split_norm(float* x, int T, int K, const float* w, float ep
                                 int ldh, float* xs, hipStream_t st, const float* part = nullptr, int nsp = 0);
 hipError_t launch_pf_split_act(const float* gu, int T, int ffn, int act, _Float16* xh, int ldh, float* xs,
                                hipStream_t st, const float* part = nullptr, int nsp = 0);
-// *out = max(*out, bits of the largest |w| over the n elements of a weight matrix in GGUF row layout)
-// (out holds a non-negative float's bits; zero it first). pf_wexp turns it into the exponent that
-// brings the matrix's largest magnitude into [2^14, 2^15) for the fp16 split.
-hipError_t launch_pf_wmax(int type, const uint8_t* w, int64_t n, unsigned* out, hipStream_t st);
+// *out = max(*out, bits of the largest magnitude that the GEMM of a weight matrix in GGUF row layout scales:
+// |dmin m| over the groups of Q4_K / Q5_K rows of whole 256-element blocks, nothing for such Q6_K rows
+// (*out stays), else |w| over the elements) (out holds a non-negative float's bits; zero it first).
+// pf_wexp turns it into the exponent that brings that magnitude into [2^14, 2^15) for the fp16 split.
+hipError_t launch_pf_wmax(int type, const uint8_t* w, int64_t rows, int64_t cols, unsigned* out, hipStream_t st);
 int pf_wexp(unsigned max_bits);
 
 // X[t] = embedding row tokens[t] (exact dequantization of any supported type)

@@ -13,7 +13,7 @@ import dotnetfoundryllm_amd as F
 import dotnetfoundryllm_amd._native as N
 import oracle_bind as O
 from dotnetfoundryllm_amd.configs import CONFIGS, desc_of, synth_bytes, tensor_plan
-from fixtures import synthetic, upload
+from fixtures import f32_of, synthetic, upload
 
 pytestmark = pytest.mark.gpu
 TOL = 1e-3
@@ -332,5 +332,38 @@ def test_prefill_gemm_tile_edges(ctx, types, hidden):
         assert O.normwise_rel_err(fwd.logits, orc.logits()) <= TOL
     finally:
         orc.close()
+        kv.close()
+        m.close()
+
+
+@pytest.mark.parametrize("top", [1e-5, 1.0, 4e3, 4e6])
+@pytest.mark.parametrize("q,v,hidden", [(N.Q4_K, N.Q4_K, 512), (N.Q5_K, N.Q5_K, 512), (N.Q8_0, N.Q5_K, 512),
+                                        (N.Q4_K, N.Q4_K, 2304), (N.Q5_K, N.Q5_K, 2304)],
+                         ids=["q4_k", "q5_k", "mixed", "q4_k-rows", "q5_k-rows"])
+def test_prefill_kquant_offset_magnitudes(ctx, q, v, hidden, top):
+    """V of a Q4_K / Q5_K matrix whose largest offset dmin m is `top`: from near the smallest half to near
+    the largest (the offsets enter the matrix cores as two halves). Bound against float64: operands of 22
+    bits and f32 sums of `hidden` products, 2^-22 + sqrt(hidden) 2^-24."""
+    cfg = dict(CONFIGS["test-llama"], n_layers=1, hidden=hidden, n_heads=8, n_kv_heads=2, head_dim=64, ffn=256, max_ctx=128,
+               types=dict(zip(("q", "k", "v", "o", "gate", "up", "down", "out"), [q, q, v] + [N.Q4_K] * 5)))
+    desc = desc_of(cfg)
+    tensors = {e[0]: (e, synth_bytes(cfg, e)) for e in tensor_plan(cfg)}
+    entry, data = tensors["blk.0.attn_v.weight"]
+    blocks = data.copy().reshape(-1, N.BLOCK[v][0])
+    mid = 7.5 if v == N.Q4_K else 15.5
+    d, dmin = np.float16(top / 63 / mid), np.float16(top / 63)  # at 1e-5 d is 0: the offsets alone
+    blocks[:, :4] = np.array([d, dmin]).view(np.uint8)
+    tensors["blk.0.attn_v.weight"] = (entry, blocks.reshape(-1))
+    m = device_model(ctx, desc, tensors)
+    kv, fwd = F.HipKvCache(m), F.HipForwardPass(m)
+    prompt = F.synth_tokens(cfg["seed"], 11, desc.vocab, 70)
+    try:
+        fwd.prefill(prompt, 0, kv)
+        x = f32_of(tensors, "token_embd.weight").astype(np.float64).reshape(-1, hidden)[prompt]
+        x = x / np.sqrt(np.mean(x * x, axis=1, keepdims=True) + 1e-5) * f32_of(tensors, "blk.0.attn_norm.weight")
+        want = x @ f32_of(tensors, "blk.0.attn_v.weight").astype(np.float64).reshape(-1, hidden).T
+        got = np.asarray(kv.get_values(0), dtype=np.float64).reshape(want.shape)
+        assert np.linalg.norm(got - want) / np.linalg.norm(want) <= 2.0**-22 + np.sqrt(hidden) * 2.0**-24
+    finally:
         kv.close()
         m.close()
