@@ -2086,13 +2086,18 @@ hipError_t launch_pack_tiles(int type, const uint8_t* src, uint8_t* dst, int64_t
 }
 
 // ---- small matrices of rows that are no whole chunks ------------------------------------------------
-// One wave per row, one 32-element group per lane and pass, exact f32 products. For matrices of at most
-// 2^21 elements and rows of at most 2048: there the launch is bound by its chain of memory latencies, and
-// k_gemv_fused's (the vector's quantization, the rows staged through LDS, 8 rows to a wave) took 8.0 us for
-// Q4_K 512 x 1408 where this one, two loads deep, takes 4.9. Longer rows read x at a stride of
-// 128 bytes per lane too often; larger matrices are bound by bytes, which the staging reads coalesced.
+// One wave per row, one 32-element group per lane and pass, a group's sum in four chains of eight f32 fmas
+// (one chain of 32 had rounded sums of inputs with a mean up to 1.6 times as far off as k_gemv_fused's
+// integers; four are closer than those. Errors over the absolute sums, k_gemv_fused, one chain, four: Q4_K
+// 1024 x 32 on inputs in [0, 1) 6.1e-8, 9.6e-8, 5.8e-8; Q8_0 512 x 352 7.8e-9, 8.8e-9, 6.5e-9).
+// For matrices of at most 2^21 elements and rows of at most 2048: there the launch is bound by its chain of
+// memory latencies, and k_gemv_fused's is longer (the vector's quantization, the rows staged through LDS,
+// 8 rows to a wave): Q4_K 512 x 1408 7.6 us, here 3.1. Over the formats: 1024 x 2048 7.3 - 8.9 us there,
+// 3.1 - 3.5 here; 4096 x 2016, past the line, 8.0 - 10.8 and 6.3 - 6.9; at 8192 x 2016 the bytes, which the
+// staging reads coalesced, have turned it: 8.6 - 12.5 and 10.2 - 11.4.
 struct __attribute__((packed, aligned(2))) Sm16 { uint32_t v[4]; };
 struct __attribute__((packed, aligned(2))) Sm8 { uint32_t v[2]; };
+__device__ __forceinline__ float sm_sum(const float* s) { return (s[0] + s[1]) + (s[2] + s[3]); }
 template <int T>
 __device__ __forceinline__ float sm_group(const uint8_t* __restrict__ w, int64_t e0, const float* x) {
     if constexpr (T == FLLM_TYPE_Q4_K || T == FLLM_TYPE_Q5_K) {
@@ -2106,50 +2111,49 @@ __device__ __forceinline__ float sm_group(const uint8_t* __restrict__ w, int64_t
         const uint32_t sc = g < 4 ? (y & 63u) : ((w4 & 15u) | ((y >> 2) & 0x30u));
         const uint32_t mn = g < 4 ? (z & 63u) : (((w4 >> 4) & 15u) | ((z >> 2) & 0x30u));
         const uint32_t q[4] = {q4.x, q4.y, q4.z, q4.w};
-        float s = 0.0f, t = 0.0f;
+        float s[4] = {}, t[4] = {};
 #pragma unroll
         for (int i = 0; i < 32; i++) {
             uint32_t c = (q[i >> 3] >> (4 * (i & 7))) & 15u;
             if constexpr (T == FLLM_TYPE_Q5_K) c |= ((hb >> i) & 1u) << 4;
-            s = fmaf((float)c, x[i], s);
-            t += x[i];
+            s[i >> 3] = fmaf((float)c, x[i], s[i >> 3]);
+            t[i >> 3] += x[i];
         }
-        return half_exact(h.x & 0xFFFFu) * (float)sc * s - half_exact(h.x >> 16) * (float)mn * t;
+        return half_exact(h.x & 0xFFFFu) * (float)sc * sm_sum(s) - half_exact(h.x >> 16) * (float)mn * sm_sum(t);
     } else if constexpr (T == FLLM_TYPE_Q6_K) {
         const uint8_t* p = w + (e0 >> 8) * 210;
         const int g = (int)((e0 & 255) >> 5);
         const Sm16 q = *(const Sm16*)(p + 16 * g);
         const Sm8 h = *(const Sm8*)(p + 128 + 8 * g);
-        float s0 = 0.0f, s1 = 0.0f;
+        float s[4] = {};
 #pragma unroll
         for (int i = 0; i < 32; i++) {
             const uint32_t c = ((q.v[i >> 3] >> (4 * (i & 7))) & 15u) | (((h.v[i >> 4] >> (2 * (i & 15))) & 3u) << 4);
-            if (i < 16) s0 = fmaf((float)((int)c - 32), x[i], s0);
-            else s1 = fmaf((float)((int)c - 32), x[i], s1);
+            s[i >> 3] = fmaf((float)((int)c - 32), x[i], s[i >> 3]);
         }
         const float d = half_exact(*(const uint16_t*)(p + 208));
-        return d * ((float)*(const int8_t*)(p + 192 + 2 * g) * s0 + (float)*(const int8_t*)(p + 193 + 2 * g) * s1);
+        return d * ((float)*(const int8_t*)(p + 192 + 2 * g) * (s[0] + s[1]) + (float)*(const int8_t*)(p + 193 + 2 * g) * (s[2] + s[3]));
     } else if constexpr (T == FLLM_TYPE_Q8_0) {
         const uint8_t* p = w + (e0 >> 5) * 34;
         const Sm16 a = *(const Sm16*)(p + 2), b = *(const Sm16*)(p + 18);
-        float s = 0.0f;
+        float s[4] = {};
 #pragma unroll
         for (int i = 0; i < 16; i++) {
-            s = fmaf((float)(int8_t)(a.v[i >> 2] >> (8 * (i & 3))), x[i], s);
-            s = fmaf((float)(int8_t)(b.v[i >> 2] >> (8 * (i & 3))), x[16 + i], s);
+            s[i >> 3] = fmaf((float)(int8_t)(a.v[i >> 2] >> (8 * (i & 3))), x[i], s[i >> 3]);
+            s[2 + (i >> 3)] = fmaf((float)(int8_t)(b.v[i >> 2] >> (8 * (i & 3))), x[16 + i], s[2 + (i >> 3)]);
         }
-        return half_exact(*(const uint16_t*)p) * s;
+        return half_exact(*(const uint16_t*)p) * sm_sum(s);
     } else {
         const uint8_t* p = w + (e0 >> 5) * 18;
         const Sm16 a = *(const Sm16*)(p + 2);
-        float s = 0.0f;
+        float s[4] = {};
 #pragma unroll
         for (int i = 0; i < 16; i++) {
             const uint32_t c = a.v[i >> 2] >> (8 * (i & 3));
-            s = fmaf((float)((int)(c & 15u) - 8), x[i], s);
-            s = fmaf((float)((int)((c >> 4) & 15u) - 8), x[16 + i], s);
+            s[i >> 3] = fmaf((float)((int)(c & 15u) - 8), x[i], s[i >> 3]);
+            s[2 + (i >> 3)] = fmaf((float)((int)((c >> 4) & 15u) - 8), x[16 + i], s[2 + (i >> 3)]);
         }
-        return half_exact(*(const uint16_t*)p) * s;
+        return half_exact(*(const uint16_t*)p) * sm_sum(s);
     }
 }
 

@@ -208,3 +208,17 @@ def test_gemv_small_matrices(ctx, t, rows, cols):
     # sums of at most 2080 f32 products: sqrt(2080) 2^-24 of the row's absolute sum, which the file's
     # bound covers for these weights
     assert O.normwise_rel_err(y, ref) <= 1e-5
+
+
+@pytest.mark.parametrize("t,bound", [(N.Q4_K, 2.0**-24), (N.Q5_K, 2.0**-24), (N.Q8_0, 2.1e-8), (N.Q4_0, 2.1e-8)])
+def test_gemv_small_matrices_rounding(ctx, t, bound):
+    """The rounding of a 32-element group's sum for inputs with a mean, as a 2-norm over the rows' absolute
+    sums. An f32 addition errs by about 2.4e-8 (rms) of its partial sum. Codes of one sign (the K-quants):
+    four chains of eight and their sum err by 2.4e-8 sqrt(4 * 204 + 2 * 16^2 + 32^2) / 32 = 3.6e-8, one
+    chain of 32 by 8e-8, and the offsets' sum adds as much again in part. Signed codes walk: 1.4e-8 to
+    1.8e-8, one chain 2.6e-8."""
+    x = (1.0 + np.random.default_rng(5).standard_normal(32)).astype(np.float32)
+    raw = synth(t, 1024 * 32, seed=3, tid=1024)
+    y, ref = run_gemv(ctx, t, 1024, 32, x=x)
+    w = O.dequantize(t, raw, 1024 * 32)[1].reshape(1024, 32).astype(np.float64)
+    assert np.linalg.norm(y - ref) <= bound * np.linalg.norm(np.abs(w) @ np.abs(x.astype(np.float64)))
