@@ -325,38 +325,43 @@ SIZE_PASSES = (("TCC_EA0_RDREQ_sum", "TCC_EA0_RDREQ_32B_sum", "TCC_EA0_RDREQ_64B
                ("TCC_BUBBLE_sum", "TCC_EA0_RDREQ_DRAM_32B_sum", "TCC_EA0_WRREQ_WRITE_DRAM_32B_sum"))
 
 
+def launches_named(order, names, want, what):
+    """The entries of order, [(kernel key, value)] of a child's dispatches, that are the launches named
+    want: the child's last kernels of this library are the profiled launches, one kernel each, in the
+    order of names (the step-parameter write before a forward is no profiled launch). One kernel can
+    serve several launches of a step with the same grid (e.g. o and gate/up), so a launch is known by its
+    position; all of one name are the same kernel, or the positions do not match."""
+    mine = [(k, v) for k, v in order if "fllm::" in k[0] and "k_set_params" not in k[0]]
+    if not names or len(mine) < len(names):
+        raise RuntimeError(f"{what}: fewer dispatches than the profiled launches")
+    kinds = {}
+    for (k, _), nm in zip(mine[-len(names):], names):
+        kinds.setdefault(nm, set()).add(k)
+    if want not in kinds or len(kinds[want]) != 1:
+        raise RuntimeError(f"{what}: the launches named {want} are the kernels {sorted(kinds.get(want, ()))}")
+    return [(k, v) for (k, v), nm in zip(mine[-len(names):], names) if nm == want]
+
+
 def profiler_roofline(args, bytes_per_launch, dom_name, steps_launches):
-    """Mean duration and HBM traffic of the dominant launch from rocprofv3 child runs. The dominant
-    launch is identified by position: the profiled steps' launches in order are the HIP-event
-    names, so the kernel (and grid) at the positions named dom_name is the dominant one."""
+    """Mean duration and HBM traffic of the dominant launch from rocprofv3 child runs, found among a
+    child's dispatches by launches_named. Raises when they cannot be that launch's: another kernel, or
+    less traffic than the launch has to read."""
     tmp = tempfile.mkdtemp(prefix="fllm_roofline_")
-    n_prof = len(steps_launches)
 
     def dominant(order, what):
-        # the dominant launch by position among the profiled launches, as for the durations (one
-        # kernel can serve several launches of a step with the same grid: e.g. o and gate/up)
-        fl = [(n, v) for n, v in order if "fllm::" in n and "k_set_params" not in n]
-        if len(fl) < n_prof:
-            raise RuntimeError(f"{what}: fewer dispatches than the profiled launches")
-        dom = [v for (n, v), nm in zip(fl[-n_prof:], steps_launches) if nm == dom_name]
-        if not dom:
-            raise RuntimeError(f"{what}: no dominant-kernel dispatches")
-        return sum(dom) / len(dom)
+        dom = launches_named([((n,), v) for n, v in order], steps_launches, dom_name, what)
+        if dom[0][0][0].split("(")[0] != symbol:
+            raise RuntimeError(f"{what}: {dom[0][0][0]} is not {symbol}")
+        return sum(v for _, v in dom) / len(dom)
 
     try:
         trace = rocprof_child(args, "trace", tmp)
         trace.sort(key=lambda r: int(r["Start_Timestamp"]))
-        # the profiled launches (one kernel each, names in order) are the child's last fllm kernels
-        # (the step-parameter write at the start of each forward is not a profiled launch)
-        mine = [r for r in trace if "fllm::" in r["Kernel_Name"] and "k_set_params" not in r["Kernel_Name"]]
-        if n_prof == 0 or len(mine) < n_prof:
-            raise RuntimeError("kernel trace shorter than the profiled launches")
-        prof = mine[-n_prof:]
-        keys = {kernel_key(r) for r, nm in zip(prof, steps_launches) if nm == dom_name}
-        durs = [int(r["End_Timestamp"]) - int(r["Start_Timestamp"]) for r, nm in zip(prof, steps_launches) if nm == dom_name]
-        avg_us = sum(durs) / len(durs) / 1e3
-        res = {"avg_launch_us": round(avg_us, 2), "duration_source": "rocprofv3 kernel trace",
-               "kernel_symbol": sorted(k[0] for k in keys)[0] if keys else None}
+        dom = launches_named([(kernel_key(r), int(r["End_Timestamp"]) - int(r["Start_Timestamp"])) for r in trace],
+                             steps_launches, dom_name, "kernel trace")
+        symbol = dom[0][0][0]
+        avg_us = sum(v for _, v in dom) / len(dom) / 1e3
+        res = {"avg_launch_us": round(avg_us, 2), "duration_source": "rocprofv3 kernel trace", "kernel_symbol": symbol}
         traffic = 0.0
         for counter in ("FETCH_SIZE", "WRITE_SIZE"):
             order = pmc_dispatches(rocprof_child(args, counter, tmp), counter)
@@ -366,6 +371,8 @@ def profiler_roofline(args, bytes_per_launch, dom_name, steps_launches):
             res[counter.lower() + "_copy_factor"] = round(factor, 4)
             traffic += kib * 1024.0 * factor
         res["traffic"] = int(traffic)
+        if traffic < 0.95 * bytes_per_launch:
+            raise RuntimeError(f"{symbol}: {traffic / 1e6:.1f} MB counted, {bytes_per_launch / 1e6:.1f} MB to read")
         try:
             sizes = {}
             for group in SIZE_PASSES:

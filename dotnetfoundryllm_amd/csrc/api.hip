@@ -1276,8 +1276,12 @@ static bool step_embed(const fllm_seq* s, StepEmb* e) {
 
 static hipError_t step_params(fllm_seq* s, int token, int pos) {
     StepEmb e;
-    return step_embed(s, &e) ? launch_set_params_embed(s->params, token, pos, s->cur_len, e, s->st)
-                             : launch_set_params(s->params, token, pos, s->cur_len, s->st);
+    if (!step_embed(s, &e)) return launch_set_params(s->params, token, pos, s->cur_len, s->st);
+    // the embedding row, then per element the norm weight, x and the table's three digits (a profiled
+    // step's first launch; the plain parameters are no work of a step and go without a name)
+    STEP("step_begin", (double)s->m->tok_embd.bytes / e.vocab + 11.0 * e.hidden,
+         launch_set_params_embed(s->params, token, pos, s->cur_len, e, s->st));
+    return hipSuccess;
 }
 
 // the greedy token of the head's n keys, and the advance to the next step; start_next: with that step's

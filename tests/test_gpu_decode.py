@@ -568,3 +568,24 @@ def test_float_projections_of_a_norm(ctx, tt, arch, hidden, ffn):
         orc.close()
         kv.close()
         m.close()
+
+
+@pytest.mark.parametrize("name", ["test-llama", "test-qwen2-qkva"])
+def test_profiled_step_names_its_start(ctx, name):
+    """The launch that begins a Forward call with the embedding row and the first table is a named launch of
+    the profiled step, its first."""
+    cfg, desc, tensors = synthetic(name)
+    m = device_model(ctx, desc, tensors)
+    kv = F.HipKvCache(m)
+    F.set_profile(kv, True)
+    fwd = F.HipForwardPass(m)
+    try:
+        for p in range(2):
+            fwd.forward(5, p, kv)
+        names = F.profile_launches(kv)
+        assert names[: len(names) // 2] == names[len(names) // 2:]
+        assert names[0] == "step_begin" and names.count("step_begin") == 2 and "embed" not in names
+        assert {e["name"]: e for e in F.profile_entries(kv)}["step_begin"]["ms"] > 0
+    finally:
+        kv.close()
+        m.close()
