@@ -1293,11 +1293,20 @@ static hipError_t step_advance(fllm_seq* s, int n, bool start_next) {
     return hipSuccess;
 }
 
-// true when the float projections of a normalized vector take these matrices in one launch
+// True when the float projections of a normalized vector take these matrices in one launch. It reads x and
+// the norm's weights again for every two rows, and streams halves at 4.3 - 4.9 TB/s where the launch of one
+// matrix reaches 5.4 - 5.9 (F32: 6.2 and 6.6), for the launches that it saves. F16 gate and up, with norm and
+// activation apart and in one: 4096 x 28672 53.4 and 48.4 us, 4096 x 32768 57.1 and 54.4, 8192 x 16384 63.0
+// and 62.9; past 2^27 elements 5120 x 27648 61.6 and 65.7, 2560 x 53248 55.9 and 61.2, 8192 x 57344 175 and
+// 201; F32 8192 x 57344 still 305 and 300. q, k and v, 8192 x 24576: 89.4 and 88.5. A single matrix saves
+// only the norm's launch, and lost (a head, 4096 x 128256: 179 and 216).
 static bool norm_gemv_launch(const Tensor* const* t, int n) {
-    for (int i = 0; i < n; i++)
+    int64_t rows = 0;
+    for (int i = 0; i < n; i++) {
         if (t[i]->layout != LAYOUT_ROWS || t[i]->type != t[0]->type || t[i]->cols != t[0]->cols) return false;
-    return norm_gemv_ok(t[0]->type, t[0]->cols);
+        rows += t[i]->rows;
+    }
+    return norm_gemv_ok(t[0]->type, t[0]->cols) && (t[0]->type == FLLM_TYPE_F32 || rows * t[0]->cols <= (int64_t)1 << 27);
 }
 static NormGemv norm_gemv_args(const fllm_seq* s, const Tensor* const* t, int n, const float* norm_w) {
     const fllm_model_desc& d = s->m->d;
@@ -1316,17 +1325,10 @@ static hipError_t head_generic(fllm_seq* s, bool start_next) {
     bool gemma = d.arch == FLLM_ARCH_GEMMA2;
     float eps = gemma ? 1e-6f : d.norm_eps;
     int H = d.hidden;
-    const Tensor* head_t[1] = {&m->output};
-    if (!s->debug && norm_gemv_launch(head_t, 1)) {
-        NormGemv a = norm_gemv_args(s, head_t, 1, m->out_norm);
-        a.out = s->logits;
-        STEP("norm_lm_head", (double)m->output.bytes + 4.0 * (2.0 * H + d.vocab), launch_norm_gemv(a, s->st));
-    } else {
-        STEP("rmsnorm", 12.0 * H, launch_rmsnorm(s->x, m->out_norm, H, eps, gemma ? 1 : 0, s->xn, s->st));
-        if (s->debug) STEP("debug_copy", 8.0 * H, launch_copy_hidden(s->xn, H, s->hidden_dbg + (size_t)d.n_layers * H, s->st));
-        hipError_t e = gemv_step(s, m->output, s->xn, s->logits, nullptr);
-        if (e != hipSuccess) return e;
-    }
+    STEP("rmsnorm", 12.0 * H, launch_rmsnorm(s->x, m->out_norm, H, eps, gemma ? 1 : 0, s->xn, s->st));
+    if (s->debug) STEP("debug_copy", 8.0 * H, launch_copy_hidden(s->xn, H, s->hidden_dbg + (size_t)d.n_layers * H, s->st));
+    hipError_t e = gemv_step(s, m->output, s->xn, s->logits, nullptr);
+    if (e != hipSuccess) return e;
     if (gemma && d.final_softcap > 0.0f) STEP("softcap", 8.0 * d.vocab, launch_softcap(s->logits, d.vocab, d.final_softcap, s->st));
     // (one kernel per profiled step: the segment keys, then their reduction and the step advance)
     STEP("argmax_segments", 4.0 * d.vocab, launch_argmax_seg(s->logits, d.vocab, s->head_keys, s->st));

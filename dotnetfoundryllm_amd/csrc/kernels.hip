@@ -153,9 +153,9 @@ hipError_t launch_gemv(const WMat& m, const float* xf, float* y, const float* re
 // =====================================================================================
 // W RmsNorm(x) = rms * W (x * w): each wave takes two rows and forms the sum of squares of x beside their dot
 // products, so the norm needs no launch of its own and no pass over x before the weights. MODE 0: rows
-// 2 p, 2 p + 1 of q | k | v (a RoPE pair); 1: row p of gate and of up; 2: rows 2 p, 2 p + 1 of one matrix.
+// 2 p, 2 p + 1 of q | k | v (a RoPE pair); 1: row p of gate and of up.
 // Bound by the weights' bytes. An F16 layer, 4096 wide, had taken norm, three projections and the RoPE /
-// store launch, then norm, gate, up and the activation: 28 and 53 us; now 12.5 and 47.8 us.
+// store launch, then norm, gate, up and the activation: 28 and 53 us; now 12.0 and 48.4 us.
 template <int T>
 __device__ __forceinline__ void fg_load(const uint8_t* __restrict__ row, int64_t v, kf_u4& u) {
     u = __builtin_nontemporal_load((const kf_u4*)row + v);
@@ -198,14 +198,10 @@ __global__ __launch_bounds__(256) void k_norm_gemv(const NormGemv a, int units) 
         const uint8_t* w = sec == 0 ? a.w[0] : sec == 1 ? a.w[1] : a.w[2];
         w0 = w + (int64_t)r0 * a.cols * ESZ;
         w1 = w0 + a.cols * ESZ;
-    } else if constexpr (MODE == 1) {
+    } else {
         r0 = p;
         w0 = a.w[0] + (int64_t)p * a.cols * ESZ;
         w1 = a.w[1] + (int64_t)p * a.cols * ESZ;
-    } else {
-        if (r1 >= a.rows[0]) r1 = r0;  // an odd last row, twice
-        w0 = a.w[0] + (int64_t)r0 * a.cols * ESZ;
-        w1 = a.w[0] + (int64_t)r1 * a.cols * ESZ;
     }
     const int64_t nvec = a.cols / PER;
     float acc0 = 0.0f, acc1 = 0.0f, ss = 0.0f;
@@ -255,11 +251,8 @@ __global__ __launch_bounds__(256) void k_norm_gemv(const NormGemv a, int units) 
             a.vc[slot + r0] = y0;
             a.vc[slot + r1] = y1;
         }
-    } else if constexpr (MODE == 1) {
-        a.out[p] = act_fn(y0, a.act) * y1;
     } else {
-        a.out[r0] = y0;
-        if (r1 != r0) a.out[r1] = y1;
+        a.out[p] = act_fn(y0, a.act) * y1;
     }
 }
 
@@ -285,7 +278,6 @@ hipError_t launch_norm_gemv_glu(const NormGemv& a, hipStream_t st) {
     if (a.rows[0] != a.rows[1]) return hipErrorInvalidValue;
     return norm_gemv<1>(a, a.rows[0], st);
 }
-hipError_t launch_norm_gemv(const NormGemv& a, hipStream_t st) { return norm_gemv<2>(a, (a.rows[0] + 1) / 2, st); }
 
 // =====================================================================================
 // Step parameters, embedding, norms

@@ -34,7 +34,7 @@ hipError_t launch_gemv_tiles(const WMat& m, const float* xf, float* y, int n_cu,
 
 // Projections of RmsNorm(x) by F32 / F16 / BF16 matrices of one type, one launch for all of them
 // (cols a multiple of 4, 2-byte types 8): q, k, v with bias, RoPE and the K / V store (even row counts and
-// head_dim); h = act(gate) * up (act 0 SiLU, 1 GELU); or plain rows (y = W RmsNorm(x)).
+// head_dim), or h = act(gate) * up (act 0 SiLU, 1 GELU).
 struct NormGemv {
     int type;
     int64_t cols;
@@ -48,7 +48,7 @@ struct NormGemv {
     const float2* rope;
     int hd;
     const StepParams* params;
-    float* out;            // q, h or y
+    float* out;            // q or h
     float* kc;             // this layer's caches [pos][rows[1]]
     float* vc;
     int act;
@@ -56,7 +56,6 @@ struct NormGemv {
 bool norm_gemv_ok(int type, int64_t cols);
 hipError_t launch_norm_gemv_qkv(const NormGemv& a, hipStream_t st);
 hipError_t launch_norm_gemv_glu(const NormGemv& a, hipStream_t st);
-hipError_t launch_norm_gemv(const NormGemv& a, hipStream_t st);
 
 hipError_t launch_set_params(StepParams* p, int token, int pos, int cur_len, hipStream_t st);
 hipError_t launch_embed(const uint8_t* emb, int type, int hidden, const StepParams* p, float* x,

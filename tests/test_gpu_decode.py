@@ -544,8 +544,8 @@ def test_greedy_runs_and_single_steps_agree(ctx, name):
 @pytest.mark.parametrize("arch,hidden,ffn", [("test-llama", 256, 264), ("test-qwen2", 264, 72), ("test-gemma2", 1032, 520)],
                          ids=["llama-256", "qwen2-264", "gemma2-1032"])
 def test_float_projections_of_a_norm(ctx, tt, arch, hidden, ffn):
-    """A model of one float type: norm + q/k/v + bias + RoPE + K/V store, norm + gate/up + activation and
-    norm + LM head as one launch each, on rows of less than, one and a half and several 64-lane loads,
+    """A model of one float type: norm + q/k/v + bias + RoPE + K/V store and norm + gate/up + activation as one
+    launch each, then norm and LM head, on rows of less than, one and a half and several 64-lane loads,
     1 + w norms and an odd vocabulary. Bound: f32 sums of at most 1032 products, sqrt(1032) 2^-24 (2e-6)
     per projection, ten in a row, the oracle's own error as large: 4e-5."""
     cfg = dict(CONFIGS[arch], n_layers=2, hidden=hidden, n_heads=4, n_kv_heads=2, head_dim=64, ffn=ffn, vocab=511,
@@ -587,5 +587,31 @@ def test_profiled_step_names_its_start(ctx, name):
         assert names[0] == "step_begin" and names.count("step_begin") == 2 and "embed" not in names
         assert {e["name"]: e for e in F.profile_entries(kv)}["step_begin"]["ms"] > 0
     finally:
+        kv.close()
+        m.close()
+
+
+@pytest.mark.parametrize("ffn,one", [(32768, True), (32776, False)], ids=["2^27", "past-2^27"])
+def test_float_projection_launches(ctx, ffn, one):
+    """Halves: norm, gate, up and activation are one launch up to 2^27 weights and separate ones past them;
+    the LM head's norm has its launch at every size. Bound: f32 sums of up to 32776 products, 2^-24
+    sqrt(32776) = 1.1e-5, the oracle's as large, through five projections."""
+    cfg = dict(CONFIGS["test-llama"], n_layers=1, hidden=2048, n_heads=4, n_kv_heads=2, head_dim=64, ffn=ffn, vocab=64,
+               max_ctx=16, tied=False, emb_type=N.F16,
+               types={k: N.F16 for k in ("q", "k", "v", "o", "gate", "up", "down", "out")})
+    desc = desc_of(cfg)
+    tensors = {e[0]: (e, synth_bytes(cfg, e)) for e in tensor_plan(cfg)}
+    m = device_model(ctx, desc, tensors)
+    kv, fwd, orc = F.HipKvCache(m), F.HipForwardPass(m), O.OracleModel(desc, tensors)
+    F.set_profile(kv, True)
+    try:
+        fwd.forward(5, 0, kv)
+        assert orc.forward(5, 0) == 0
+        names = F.profile_launches(kv)
+        assert ("norm_gate_up_act" in names) == one and ("ffn_act" in names) == (not one)
+        assert "norm_qkv_rope_kv" in names and "norm_lm_head" not in names
+        assert O.normwise_rel_err(fwd.logits, orc.logits()) <= 1.2e-4
+    finally:
+        orc.close()
         kv.close()
         m.close()
