@@ -15,9 +15,12 @@
 //  - Q8_0, Q4_0: the code (Q4_0: minus 8), exact; two MFMAs, each 32-element block's sum scaled by its d.
 //  - F16: the weight itself times a power of two that costs no bit; two MFMAs.
 //
-// The MFMA rounds its sums down (a -7e-8 of the result's root mean square, the same for every output, was
-// measured in the Q8_0 form): every other block (step, in the step-scaled forms) enters with its codes and
-// its d negated, so that half of the sums err upwards.
+// The MFMA rounds its sums down, the same way for every output (Q8_0, 2048 columns: -4e-8 of the result's root
+// mean square): in the forms of codes every other block (step, in the step-scaled forms) enters with its codes
+// and its d negated, so that half of the sums err upwards (below 5e-9 since). Not in F16, whose total stays in
+// the MFMA: -1.6e-8 at 2048 columns, -4e-8 at 8192, as its three products had; a total beside the block's sum
+// ran 3.5% longer, one negated in place 2% (4096 wide, 2000 tokens). Nor do the min terms alternate, which
+// enter the total by one MFMA a block: 6e-10 of Q4_K at 8192 columns.
 //
 // What bounds it: the matrix cores beside the card's power. A tile of 64 tokens x 128 rows on four waves
 // (32 x 64 each, three workgroups per CU, one LDS stage, two barriers a step) issued 5.2 vector-ALU
