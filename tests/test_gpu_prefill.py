@@ -293,8 +293,8 @@ def test_prefill_argument_contract(ctx):
     ids=["q4_k", "q5_k", "q6_k", "q8_0", "mixed", "q4_k-rows", "q5_k-rows", "q6_k-rows", "q8_0-rows", "q4_0", "f16",
          "q4_0-352"])
 def test_prefill_gemm_tile_edges(ctx, types, hidden):
-    """The large-tile GEMMs at the edges of their tiles (64 and 128 tokens x 256 weight rows): 2 to
-    200 tokens on 128-, 512- and 768-row matrices, every tile-interleaved type alone, launches that mix
+    """The large-tile GEMMs at the edges of the tiles of 64 tokens x 256 weight rows: 2 to
+    200 tokens on 128-, 512- and 768-row matrices (at most 24 such tiles: never the ones of 128 tokens), every tile-interleaved type alone, launches that mix
     them, and GGUF rows (2304 = 9 blocks has no tile layout, Q4_0 and F16 none at all; 352 is no whole
     number of blocks and stays on the general row kernel). K / V rows of both layers (the second
     layer's carry every GEMM of the first) against the oracle. Bound: operands of 22 bits or more and
@@ -392,6 +392,60 @@ def test_prefill_gemm_rounds_without_bias(ctx, t, hidden):
         want = x @ f32_of(tensors, "blk.0.attn_v.weight").astype(np.float64).reshape(-1, hidden).T
         got = np.asarray(kv.get_values(0), dtype=np.float64).reshape(want.shape)
         assert abs(np.mean(got - want)) <= 6e-9 * np.sqrt(np.mean(want * want))
+    finally:
+        kv.close()
+        m.close()
+
+
+@pytest.mark.parametrize("gate,up,hidden,ffn,lengths", [
+    ("q4_k", "q4_k", 512, 8480, (193, 256, 257, 300)), ("q5_k", "q5_k", 512, 8480, (193, 257)),
+    ("q6_k", "q6_k", 512, 8480, (193, 257)), ("q8_0", "q8_0", 512, 8480, (193, 257)),
+    ("q5_k", "q8_0", 512, 8480, (193, 257)), ("q8_0", "q4_k", 512, 8480, (193, 257)), ("q6_k", "q5_k", 512, 8480, (193, 257)),
+    ("q4_k", "q4_k", 2304, 8480, (193, 257)), ("q5_k", "q5_k", 2304, 8480, (193, 257)),
+    ("q6_k", "q6_k", 2304, 8480, (193, 257)), ("q8_0", "q8_0", 2304, 8480, (193, 257)),
+    ("q4_0", "q4_0", 512, 8480, (193, 256, 257, 300)), ("f16", "f16", 512, 8480, (193, 257)),
+    ("q4_k", "q4_k", 8192, 8192, (256,)), ("q4_0", "q4_0", 5632, 8192, (256,))],
+    ids=["q4_k", "q5_k", "q6_k", "q8_0", "q5_k+q8_0", "q8_0+q4_k", "q6_k+q5_k", "q4_k-rows", "q5_k-rows", "q6_k-rows",
+         "q8_0-rows", "q4_0", "f16", "q4_k-split", "q4_0-split"])
+def test_prefill_gemm_tiles_of_128_tokens(ctx, gate, up, hidden, ffn, lengths):
+    """Gate / up launches that take the tiles of 128 tokens x 256 rows by the modelled time: 2 x 8480 rows are
+    68 column tiles, 193 to 256 tokens then 272 tiles of 64 tokens (two waves of 256) or 136 of 128 (one), 257
+    to 300 tokens 340 or 204; a last tile of one token, of 65, of 44 and a full one, 32 rows in each segment's
+    last tile. 2 x 8192 rows of 22 or 32 blocks over 256 tokens run in two parts of K. Each form alone and mixed.
+    The output projection is zero, so V of the second layer is a function of the first layer's FFN. Bound
+    against float64: three projections of operands of 22 bits and f32 sums of at most 8480 products,
+    3 (2^-22 + sqrt(8480) 2^-24)."""
+    name_of = {"q4_k": N.Q4_K, "q5_k": N.Q5_K, "q6_k": N.Q6_K, "q8_0": N.Q8_0, "q4_0": N.Q4_0, "f16": N.F16}
+    cfg = dict(CONFIGS["test-llama"], n_layers=2, hidden=hidden, n_heads=4, n_kv_heads=2, head_dim=64, ffn=ffn, max_ctx=320,
+               vocab=512, types=dict(zip(("q", "k", "v", "o", "gate", "up", "down", "out"),
+                                         [N.Q8_0] * 4 + [name_of[gate], name_of[up]] + [N.Q8_0] * 2)))
+    desc = desc_of(cfg)
+    tensors = {e[0]: (e, synth_bytes(cfg, e)) for e in tensor_plan(cfg)}
+    for l in range(2):
+        e, data = tensors[f"blk.{l}.attn_output.weight"]
+        tensors[f"blk.{l}.attn_output.weight"] = (e, np.zeros_like(data))
+
+    def mul(x, name):
+        return x @ f32_of(tensors, name).astype(np.float64).reshape(-1, x.shape[1]).T
+
+    def norm(x, name):
+        return x / np.sqrt(np.mean(x * x, axis=1, keepdims=True) + 1e-5) * f32_of(tensors, name)
+
+    m = device_model(ctx, desc, tensors)
+    kv, fwd = F.HipKvCache(m), F.HipForwardPass(m)
+    prompt = F.synth_tokens(cfg["seed"], 7, desc.vocab, max(lengths))
+    try:
+        x = f32_of(tensors, "token_embd.weight").astype(np.float64).reshape(-1, hidden)[prompt]
+        xn = norm(x, "blk.0.ffn_norm.weight")
+        g = mul(xn, "blk.0.ffn_gate.weight")
+        x = x + mul(g / (1.0 + np.exp(-np.clip(g, -700, 700))) * mul(xn, "blk.0.ffn_up.weight"), "blk.0.ffn_down.weight")
+        want = mul(norm(x, "blk.1.attn_norm.weight"), "blk.1.attn_v.weight")
+        for n in lengths:
+            kv.clear()
+            fwd.prefill(prompt[:n], 0, kv)
+            got = np.asarray(kv.get_values(1), dtype=np.float64).reshape(n, -1)
+            err = np.linalg.norm(got - want[:n], axis=1) / np.linalg.norm(want[:n], axis=1)
+            assert err.max() <= 3 * (2.0**-22 + np.sqrt(8480) * 2.0**-24), (n, int(err.argmax()), err.max())
     finally:
         kv.close()
         m.close()
