@@ -1823,8 +1823,7 @@ static hipError_t pf_gemm(fllm_seq* s, const char* name, const Tensor* const* w,
     }
     double bytes = 0.0;
     for (int i = 0; i < n; i++) {
-        // one launch per run of tile-interleaved matrices, or of GGUF-row matrices of one type (a run
-        // of tile Q4_K matrices only takes their own fp16 form; a mixed run, the general one)
+        // one launch per run of tile-interleaved matrices (of any types), or of GGUF-row matrices of one type
         const bool split = g.nseg > 0 && ((w[i]->layout == LAYOUT_TILES) != (g.seg[0].layout == LAYOUT_TILES) ||
                                           (w[i]->layout != LAYOUT_TILES && w[i]->type != g.seg[0].type));
         if (split) {

@@ -1,6 +1,6 @@
 // pf_gemm8.hip — the prefill GEMMs of tile-interleaved Q4_K / Q5_K / Q6_K / Q8_0 weights and of GGUF rows
-// of whole 256-element blocks (those types, Q4_0 and F16): workgroups of eight waves (2 along the tokens x 4 along the weight rows), each 32 TI tokens x 64 weight rows, so
-// tiles of 64 or 128 tokens x 256 rows.
+// of whole 256-element blocks (those types, Q4_0 and F16): workgroups of eight waves (2 along the tokens x 4
+// along the weight rows), each 32 TI tokens x 64 weight rows, so tiles of 64 or 128 tokens x 256 rows.
 //
 // Numerics: fp16 matrix cores on X's two planes (22 bits) and on exact integers of the weights:
 //  - Q4_K, Q5_K: w = d (sc q) - dmin m; sc q is an integer below 2048, exact in fp16, so a product is two
@@ -164,7 +164,7 @@ template <> struct G8W<FLLM_TYPE_Q6_K> {
         r.qh = g8_ld2(w, o + 16 * n + 2 * c, s + 2048 + 256 * (g & 3) + (g < 4 ? 0 : 8));
         r.sc = g8_ld1(w, o + 4 * n + (c >> 1), s + 3072 + 64 * (g & 3) + (g < 4 ? 0 : 2));
     }
-    // hi and lo halves of the exact integer sc q (pf_q6_pairs)
+    // hi and lo halves of the exact integer sc q
     __device__ static void decode2(const Raw& r, float sign, g8_u4& hi, g8_u4& lo) {
         const _Float16 s = (_Float16)(sign * (float)r.sc);
         const g8_h2 sc2 = {s, s}, off = {(_Float16)-1056.0f, (_Float16)-1056.0f};

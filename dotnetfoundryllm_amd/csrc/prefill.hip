@@ -78,7 +78,6 @@ __device__ __forceinline__ void pf_wave_sync() {
 }
 
 // ---- exact dequantization of 32 weights [k0, k0 + 32) of row r (k0 a multiple of 32) -----------
-// load() fetches the raw bytes of the group (issued a K step ahead), deq() decodes them.
 template <int WT> struct PfW;
 
 // GGUF rows: elements e0 = r * K + k0 .. e0 + 31 of the flat block stream (K % 32 == 0, so the
@@ -88,9 +87,7 @@ template <int WT> struct PfW;
 constexpr int PF_ROWS = 100;
 
 template <> struct PfW<-1> {
-    struct Raw {};
-    __device__ static void load(Raw&, const uint8_t*, int, int, int) {}
-    __device__ static void deq(const Raw&, const uint8_t* __restrict__ w, int type, int K, int r, int k0, float* v, float s = 1.0f) {
+    __device__ static void deq(const uint8_t* __restrict__ w, int type, int K, int r, int k0, float* v, float s = 1.0f) {
         const int64_t e0 = (int64_t)r * K + k0;
         for (int i = 0; i < 32; i++) v[i] = deq_elem(type, w, e0 + i) * s;
     }
@@ -98,9 +95,7 @@ template <> struct PfW<-1> {
 
 // Q8_0 (Dequantizer.cs:203-231): (sbyte)q * d, one 34-byte block per group
 template <> struct PfW<PF_ROWS + FLLM_TYPE_Q8_0> {
-    struct Raw {};
-    __device__ static void load(Raw&, const uint8_t*, int, int, int) {}
-    __device__ static void deq(const Raw&, const uint8_t* __restrict__ w, int, int K, int r, int k0, float* v, float s = 1.0f) {
+    __device__ static void deq(const uint8_t* __restrict__ w, int, int K, int r, int k0, float* v, float s = 1.0f) {
         const uint8_t* p = w + (((int64_t)r * K + k0) >> 5) * 34;
         const float d = half_exact(deq_ld_u16(p)) * s;
 #pragma unroll
@@ -110,9 +105,7 @@ template <> struct PfW<PF_ROWS + FLLM_TYPE_Q8_0> {
 
 // Q4_0 (Dequantizer.cs:155-185): (nibble - 8) * d, low nibbles are elements 0..15
 template <> struct PfW<PF_ROWS + FLLM_TYPE_Q4_0> {
-    struct Raw {};
-    __device__ static void load(Raw&, const uint8_t*, int, int, int) {}
-    __device__ static void deq(const Raw&, const uint8_t* __restrict__ w, int, int K, int r, int k0, float* v, float s = 1.0f) {
+    __device__ static void deq(const uint8_t* __restrict__ w, int, int K, int r, int k0, float* v, float s = 1.0f) {
         const uint8_t* p = w + (((int64_t)r * K + k0) >> 5) * 18;
         const float d = half_exact(deq_ld_u16(p)) * s;
 #pragma unroll
@@ -126,9 +119,7 @@ template <> struct PfW<PF_ROWS + FLLM_TYPE_Q4_0> {
 
 // Q4_K (Dequantizer.cs:251-294) in GGUF rows
 template <> struct PfW<PF_ROWS + FLLM_TYPE_Q4_K> {
-    struct Raw {};
-    __device__ static void load(Raw&, const uint8_t*, int, int, int) {}
-    __device__ static void deq(const Raw&, const uint8_t* __restrict__ w, int, int K, int r, int k0, float* v, float s = 1.0f) {
+    __device__ static void deq(const uint8_t* __restrict__ w, int, int K, int r, int k0, float* v, float s = 1.0f) {
         const int64_t e0 = (int64_t)r * K + k0;
         const uint8_t* p = w + (e0 >> 8) * 144;
         const int g = (int)((e0 & 255) >> 5);
@@ -150,9 +141,7 @@ template <> struct PfW<PF_ROWS + FLLM_TYPE_Q4_K> {
 
 // Q5_K (Dequantizer.cs:316-368): low nibble from qs, bit 4 from qh[t >> 3] bit (t & 7)
 template <> struct PfW<PF_ROWS + FLLM_TYPE_Q5_K> {
-    struct Raw {};
-    __device__ static void load(Raw&, const uint8_t*, int, int, int) {}
-    __device__ static void deq(const Raw&, const uint8_t* __restrict__ w, int, int K, int r, int k0, float* v, float s = 1.0f) {
+    __device__ static void deq(const uint8_t* __restrict__ w, int, int K, int r, int k0, float* v, float s = 1.0f) {
         const int64_t e0 = (int64_t)r * K + k0;
         const uint8_t* p = w + (e0 >> 8) * 176;
         const int t0 = (int)(e0 & 255), g = t0 >> 5;
@@ -176,9 +165,7 @@ template <> struct PfW<PF_ROWS + FLLM_TYPE_Q5_K> {
 
 // Q6_K (Dequantizer.cs:378-417) in GGUF rows
 template <> struct PfW<PF_ROWS + FLLM_TYPE_Q6_K> {
-    struct Raw {};
-    __device__ static void load(Raw&, const uint8_t*, int, int, int) {}
-    __device__ static void deq(const Raw&, const uint8_t* __restrict__ w, int, int K, int r, int k0, float* v, float s = 1.0f) {
+    __device__ static void deq(const uint8_t* __restrict__ w, int, int K, int r, int k0, float* v, float s = 1.0f) {
         const int64_t e0 = (int64_t)r * K + k0;
         const uint8_t* p = w + (e0 >> 8) * 210;
         const int i0 = (int)(e0 & 255);
@@ -201,27 +188,21 @@ template <> struct PfW<PF_ROWS + FLLM_TYPE_Q6_K> {
 
 // F16 / BF16 / F32 rows: exact widening (Dequantizer.cs:68-137)
 template <> struct PfW<PF_ROWS + FLLM_TYPE_F32> {
-    struct Raw {};
-    __device__ static void load(Raw&, const uint8_t*, int, int, int) {}
-    __device__ static void deq(const Raw&, const uint8_t* __restrict__ w, int, int K, int r, int k0, float* v, float s = 1.0f) {
+    __device__ static void deq(const uint8_t* __restrict__ w, int, int K, int r, int k0, float* v, float s = 1.0f) {
         const uint8_t* p = w + ((int64_t)r * K + k0) * 4;
 #pragma unroll
         for (int i = 0; i < 32; i++) v[i] = bits_f32(deq_ld_u32(p + 4 * i)) * s;
     }
 };
 template <> struct PfW<PF_ROWS + FLLM_TYPE_F16> {
-    struct Raw {};
-    __device__ static void load(Raw&, const uint8_t*, int, int, int) {}
-    __device__ static void deq(const Raw&, const uint8_t* __restrict__ w, int, int K, int r, int k0, float* v, float s = 1.0f) {
+    __device__ static void deq(const uint8_t* __restrict__ w, int, int K, int r, int k0, float* v, float s = 1.0f) {
         const uint8_t* p = w + ((int64_t)r * K + k0) * 2;
 #pragma unroll
         for (int i = 0; i < 32; i++) v[i] = half_exact(deq_ld_u16(p + 2 * i)) * s;
     }
 };
 template <> struct PfW<PF_ROWS + FLLM_TYPE_BF16> {
-    struct Raw {};
-    __device__ static void load(Raw&, const uint8_t*, int, int, int) {}
-    __device__ static void deq(const Raw&, const uint8_t* __restrict__ w, int, int K, int r, int k0, float* v, float s = 1.0f) {
+    __device__ static void deq(const uint8_t* __restrict__ w, int, int K, int r, int k0, float* v, float s = 1.0f) {
         const uint8_t* p = w + ((int64_t)r * K + k0) * 2;
 #pragma unroll
         for (int i = 0; i < 32; i++) v[i] = bf16_exact(deq_ld_u16(p + 2 * i)) * s;
@@ -229,10 +210,9 @@ template <> struct PfW<PF_ROWS + FLLM_TYPE_BF16> {
 };
 
 // ---- GEMM ---------------------------------------------------------------------------------------
-// Workgroup tile: BM tokens (64 in every launch) x 128 weight rows, 4 waves in a 2 x 2 arrangement, each
-// (BM / 2) x 64 (BM / 32 x 4 MFMA tiles of 16 x 16). Per K step of 64 the workgroup stages X and the
-// decoded weights into LDS.
-constexpr int PF_BN = 128, PF_BK = 64;
+// Workgroup tile: PF_BM tokens x PF_BN weight rows, 4 waves in a 2 x 2 arrangement, each 32 x 64 (2 x 4
+// MFMA tiles of 16 x 16). Per K step of 64 the workgroup stages X and the decoded weights into LDS.
+constexpr int PF_BM = 64, PF_BN = 128, PF_BK = 64;
 
 // workgroup (x, y): column tile x of the launch's segments, token tile y
 __device__ __forceinline__ int pf_seg_of(const PfGemm& a, int& bx) {
@@ -254,10 +234,7 @@ constexpr int PF_LDH = PF_BK + 16;
 typedef _Float16 pf_h8 __attribute__((ext_vector_type(8)));
 typedef _Float16 pf_hv2 __attribute__((ext_vector_type(2)));
 
-template <int BM>
-static constexpr size_t pf_gemm_lds_h() {
-    return sizeof(_Float16) * 2 * (size_t)(BM + PF_BN) * PF_LDH;
-}
+constexpr size_t PF_LDS_H = sizeof(_Float16) * 2 * (size_t)(PF_BM + PF_BN) * PF_LDH;
 
 // hi / lo halves of 8 scaled values, two at a time with the packed round-toward-zero conversion:
 // hi keeps 11 bits of each value, lo the remainder (exact in f32) to 11 bits
@@ -275,13 +252,13 @@ __device__ __forceinline__ void pf_split8(const float* v, uint4& hi, uint4& lo) 
     lo = make_uint4(l[0], l[1], l[2], l[3]);
 }
 
-// Tile: BM tokens x 128 weight rows, 4 waves of (BM / 2) x 64, K steps of 64.
 // MFMA 16x16x32 f16: lane l supplies row (l & 15) of the A (tokens) and B (weight rows) tiles with
 // k = 8 (l >> 4) .. + 7 of a 32-wide slice, one 16-byte LDS read per operand and plane; D lane l holds
 // rows 4 (l >> 4) .. + 3 of column l & 15.
-template <int WT, int BM>
+template <int WT>
 __device__ __forceinline__ void pf_gemm_tile_h(const PfGemm& a, const PfSeg& sg, int n0, int t0, _Float16* sx,
                                                _Float16* sw) {
+    constexpr int BM = PF_BM;
     constexpr int WM = BM / 2;   // tokens per wave
     constexpr int TI = WM / 16;  // MFMA tiles along the tokens
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -299,9 +276,7 @@ __device__ __forceinline__ void pf_gemm_tile_h(const PfGemm& a, const PfSeg& sg,
     const int wrow = tid & (PF_BN - 1), wgrp = tid / PF_BN, wr = n0 + wrow;
     const bool wlive = wr < sg.N;
     const float wsc = ldexpf(1.0f, -sg.wexp);
-    using Raw = typename PfW<WT>::Raw;
     uint4 xr[XP];
-    Raw wraw;
     auto fetch = [&](int k0) {
 #pragma unroll
         for (int i = 0; i < XP; i++) {
@@ -310,7 +285,6 @@ __device__ __forceinline__ void pf_gemm_tile_h(const PfGemm& a, const PfSeg& sg,
             xr[i] = (t < a.T && k < a.K) ? *(const uint4*)(a.xh + pl * plane + (size_t)t * a.ldh + k)
                                          : make_uint4(0u, 0u, 0u, 0u);
         }
-        if (wlive && k0 + 32 * wgrp < a.K) PfW<WT>::load(wraw, sg.w, a.K, wr, k0 + 32 * wgrp);
     };
     const int kb = (int)blockIdx.z * a.kpart, ke = kb + a.kpart < a.K ? kb + a.kpart : a.K;
     fetch(kb);
@@ -325,7 +299,7 @@ __device__ __forceinline__ void pf_gemm_tile_h(const PfGemm& a, const PfSeg& sg,
             float v[32];
             const int k = k0 + 32 * wgrp;
             if (wlive && k < a.K) {
-                PfW<WT>::deq(wraw, sg.w, sg.type, a.K, wr, k, v, wsc);
+                PfW<WT>::deq(sg.w, sg.type, a.K, wr, k, v, wsc);
             } else {
 #pragma unroll
                 for (int i = 0; i < 32; i++) v[i] = 0.0f;
@@ -340,7 +314,7 @@ __device__ __forceinline__ void pf_gemm_tile_h(const PfGemm& a, const PfSeg& sg,
                 *(uint4*)(d1 + 8 * i) = lo;
             }
         }
-        // the next step's global loads fly while this step multiplies
+        // the next step's X loads fly while this step multiplies
         if (k0 + PF_BK < ke) fetch(k0 + PF_BK);
         __syncthreads();
 #pragma unroll
@@ -399,12 +373,12 @@ __device__ __forceinline__ void pf_gemm_tile_h(const PfGemm& a, const PfSeg& sg,
         }
 }
 
-template <int BM, int RT>
+template <int RT>
 __global__ __launch_bounds__(256) void k_pf_gemm_rows_h(const PfGemm a) {
     extern __shared__ __attribute__((aligned(16))) _Float16 pf_ldh[];
     int bx = blockIdx.x;
     const int si = pf_seg_of(a, bx);
-    pf_gemm_tile_h<RT, BM>(a, a.seg[si], bx * PF_BN, blockIdx.y * BM, pf_ldh, pf_ldh + (size_t)2 * BM * PF_LDH);
+    pf_gemm_tile_h<RT>(a, a.seg[si], bx * PF_BN, blockIdx.y * PF_BM, pf_ldh, pf_ldh + (size_t)2 * PF_BM * PF_LDH);
 }
 
 // row t of X: the power of two bringing its largest magnitude into [2^14, 2^15), then the hi / lo
@@ -493,7 +467,11 @@ hipError_t launch_pf_split(const float* x, int ldx, int T, int K, _Float16* xh, 
 // sum; SRC 1 writes it back to x.
 // One workgroup of NW waves per row. 37 rows of 4096 with 15 slices: 16.0 us with 4 waves and one slice
 // load at a time, 6.4 with 16 waves and four.
-// rows up to which a row-wise kernel spreads each row over 16 waves (two rows per CU)
+// rows up to which a row-wise kernel spreads each row over 16 waves (two rows per CU of 256). 16 waves and 4,
+// us: the norm form, 4096 wide, 256 rows 8.7 and 10.9, 512 11.6 and 11.3, 640 12.8 and 11.4; 3584 wide 512
+// 5.8 and 6.9, 640 8.2 and 7.0; the post-norm, 3584 wide, 512 9.6 and 11.0, 640 13.1 and 11.3. The qkv
+// post-processing turns later (a workgroup per 256 pairs of a row, and one per row: 512 rows 9.0 and 12.8, 768
+// 14.7 and 17.9, 1024 12.8 and 11.6) and keeps the same line.
 constexpr int PF_FEW_ROWS = 512;
 template <int NPT, int SRC, int NW>
 __global__ __launch_bounds__(64 * NW) void k_pf_split_src(float* __restrict__ x, int ldx, int K,
@@ -723,18 +701,17 @@ __global__ __launch_bounds__(256) void k_pf_split_add(float* __restrict__ y, con
 }
 
 
-template <int BM>
 static PfGemmKernel pf_rows_kernel_h(int type) {
     switch (type) {
-        case FLLM_TYPE_Q8_0: return k_pf_gemm_rows_h<BM, PF_ROWS + FLLM_TYPE_Q8_0>;
-        case FLLM_TYPE_Q4_0: return k_pf_gemm_rows_h<BM, PF_ROWS + FLLM_TYPE_Q4_0>;
-        case FLLM_TYPE_Q4_K: return k_pf_gemm_rows_h<BM, PF_ROWS + FLLM_TYPE_Q4_K>;
-        case FLLM_TYPE_Q5_K: return k_pf_gemm_rows_h<BM, PF_ROWS + FLLM_TYPE_Q5_K>;
-        case FLLM_TYPE_Q6_K: return k_pf_gemm_rows_h<BM, PF_ROWS + FLLM_TYPE_Q6_K>;
-        case FLLM_TYPE_F32: return k_pf_gemm_rows_h<BM, PF_ROWS + FLLM_TYPE_F32>;
-        case FLLM_TYPE_F16: return k_pf_gemm_rows_h<BM, PF_ROWS + FLLM_TYPE_F16>;
-        case FLLM_TYPE_BF16: return k_pf_gemm_rows_h<BM, PF_ROWS + FLLM_TYPE_BF16>;
-        default: return k_pf_gemm_rows_h<BM, -1>;
+        case FLLM_TYPE_Q8_0: return k_pf_gemm_rows_h<PF_ROWS + FLLM_TYPE_Q8_0>;
+        case FLLM_TYPE_Q4_0: return k_pf_gemm_rows_h<PF_ROWS + FLLM_TYPE_Q4_0>;
+        case FLLM_TYPE_Q4_K: return k_pf_gemm_rows_h<PF_ROWS + FLLM_TYPE_Q4_K>;
+        case FLLM_TYPE_Q5_K: return k_pf_gemm_rows_h<PF_ROWS + FLLM_TYPE_Q5_K>;
+        case FLLM_TYPE_Q6_K: return k_pf_gemm_rows_h<PF_ROWS + FLLM_TYPE_Q6_K>;
+        case FLLM_TYPE_F32: return k_pf_gemm_rows_h<PF_ROWS + FLLM_TYPE_F32>;
+        case FLLM_TYPE_F16: return k_pf_gemm_rows_h<PF_ROWS + FLLM_TYPE_F16>;
+        case FLLM_TYPE_BF16: return k_pf_gemm_rows_h<PF_ROWS + FLLM_TYPE_BF16>;
+        default: return k_pf_gemm_rows_h<-1>;
     }
 }
 
@@ -799,7 +776,7 @@ hipError_t launch_pf_gemm(PfGemm a, int n_cu, hipStream_t st, int* pending) {
     if (tiles && !big) return hipErrorInvalidValue;
     for (int c = 0; c < (big ? 2 : 1); c++) {
         const PfKernel kc = big ? pf_gemm8_kernel(form, c == 0 ? 64 : 128)
-                                : PfKernel{pf_rows_kernel_h<64>(a.seg[0].type), pf_gemm_lds_h<64>(), 64, PF_BN, 256, 0.0};
+                                : PfKernel{pf_rows_kernel_h(a.seg[0].type), PF_LDS_H, PF_BM, PF_BN, 256, 0.0};
         hipError_t e = pf_lds_attr((const void*)kc.k, kc.lds);
         if (e != hipSuccess) return e;
         int64_t ct = 0;

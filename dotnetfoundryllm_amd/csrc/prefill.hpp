@@ -18,7 +18,7 @@ struct PfSeg {
     int N;
     float* y;   // [T][ldy], column 0 = weight row 0
     int ldy;
-    int tiles;  // set by launch_pf_gemm: 128-row column tiles of the segment
+    int tiles;  // set by launch_pf_gemm: column tiles of the segment (of its kernel's 128 or 256 rows)
     int wexp;   // fp16 matrix cores: the weights (Q4_K / Q5_K rows of whole blocks: the offsets dmin m) enter
                 // scaled by 2^-wexp (launch_pf_wmax gives it)
 };
