@@ -1568,7 +1568,9 @@ static hipError_t enqueue_body(fllm_seq* s, bool start_next) {
 
 // Steps of the greedy loop captured together: about 8 us pass between two graph launches (Llama 4096
 // wide, two layers: 107 us of kernels in a step of 115), paid once per run. A run's graph costs about 100
-// us to make, the gain of four runs: it is made once a sequence has taken that many steps one by one.
+// us to make at two layers, the gain of four runs: it is made once a sequence has taken that many steps one by
+// one. Fresh sequences against one graph per step that starts nothing (and k_argmax_keys): 2048 wide, 64 steps,
+// two layers 5941 and 5471 us, 24 layers 56.4 and 56.0 ms; 4096 wide, 32 layers, 32 steps 47.3 and 46.9 ms.
 constexpr int GREEDY_RUN = 4, GREEDY_RUN_AFTER = 16;
 
 // replay of captured steps (captured first when they are not); the parameters are set

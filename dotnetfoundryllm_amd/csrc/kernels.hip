@@ -682,7 +682,7 @@ hipError_t launch_argmax_keys(const unsigned long long* keys, int n, StepParams*
 // belong to (StepEmb). One workgroup, bound by latency: two dependent memory round trips (the token's keys,
 // then its row; the norm weights are loaded beside the keys). The first projection of a step had read
 // the embedding row and built the table in each of its workgroups, 9.0 us more than from a table
-// (Llama 4096 wide: 15.8 and 6.9 us); this launch takes 5.5 us where k_argmax_keys took 4.0.
+// (Llama 4096 wide: 15.8 and 6.9 us); this launch takes 6.0 us where k_argmax_keys takes 3.5.
 template <bool KEYS>
 __global__ __launch_bounds__(1024) void k_step_begin(const unsigned long long* __restrict__ keys, int n, StepParams* p,
                                                      int* tokens_out, int tokens_cap, int token, int pos, int cur_len,

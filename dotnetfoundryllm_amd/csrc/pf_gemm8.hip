@@ -296,6 +296,10 @@ template <> struct G8W<PF_FORM_ROWS + FLLM_TYPE_F16> {
 // so no product overflows and every value, a subnormal one too, keeps its bits; never down (e >= 0)
 __device__ __forceinline__ int g8_f16_exp(int wexp) { return wexp > 0 ? 0 : wexp < -30 ? 30 : -wexp; }
 
+// 2^e for |e| <= 126, in scalar registers where e is (wexp is the segment's; a ldexpf holds a vector register
+// through the loop)
+__device__ __forceinline__ float g8_pow2(int e) { return __uint_as_float((uint32_t)(127 + e) << 23); }
+
 // ---- tile ---------------------------------------------------------------------------------------
 // LDS of a tile of BM tokens x BN rows: two stages of [X hi | X lo | W planes] rows of 32 halves
 // (16-byte chunk c of row r at position c ^ ((r >> 2) & 2): a 16-row operand read is then free of
@@ -320,7 +324,7 @@ __device__ __forceinline__ void g8_tile(const PfGemm& a, const PfSeg& sg, int n0
     _Float16* sav = lds + 2 * STAGE;                               // MIN: [BM][G8_LDV]
     _Float16* swv = sav + (MIN ? BM * G8_LDV : 0);                 // MIN: [BN][G8_LDV]
     float* sd = (float*)(swv + (MIN ? BN * G8_LDV : 0));           // d: [BN] of the block, Q8_0 [2][BN] of the step
-    float* sxs = sd + 2 * BN;                                      // the tokens' factors xs
+    float* sxs = sd + 2 * BN;                                      // what undoes the scales: the tokens' xs times the weights'
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int wm = wave >> 2, wn = wave & 3;
 
@@ -349,8 +353,8 @@ __device__ __forceinline__ void g8_tile(const PfGemm& a, const PfSeg& sg, int n0
     }
     // row r0 + 128 i of a stage: the swizzle depends on r0 alone
     const int so = r0 * G8_BK + ((ch ^ ((r0 >> 2) & 2)) << 3);
-    const float wsc = ldexpf(1.0f, -sg.wexp);
-    const float msc = MIN ? wsc * 0.015625f : 1.0f;  // what the sums of the block-scaled forms are held times
+    const float wsc = g8_pow2(-sg.wexp);  // |wexp| <= 120 (pf_wexp)
+    const float msc = MIN ? g8_pow2(-sg.wexp - 6) : 1.0f;  // what the sums of the block-scaled forms are held times
     const int fe = F16 ? g8_f16_exp(sg.wexp) : 0;
     const _Float16 fh0 = (_Float16)ldexpf(1.0f, fe < 15 ? fe : 15), fh1 = (_Float16)ldexpf(1.0f, fe < 15 ? 0 : fe - 15);
     const g8_h2 fs0 = {fh0, fh0}, fs1 = {fh1, fh1};
@@ -412,7 +416,8 @@ __device__ __forceinline__ void g8_tile(const PfGemm& a, const PfSeg& sg, int n0
 #pragma unroll
         for (int j = 0; j < 4; j++) acc[i][j] = blk[i][j] = zero;
 
-    if (tid < BM) sxs[tid] = a.xs[t0 + tid < a.T ? t0 + tid : a.T - 1];
+    const float wun = F16 ? g8_pow2(-fe) : SC == G8_SC_STEP ? g8_pow2(sg.wexp) : MIN ? g8_pow2(sg.wexp + 6) : 1.0f;
+    if (tid < BM) sxs[tid] = a.xs[t0 + tid < a.T ? t0 + tid : a.T - 1] * wun;
     float sign = 1.0f;  // of the current block's codes and d: every other block enters negated
     load_b(blk_c, b0);
     if (MIN && vt < BM) xv = g8_ld16(vb, vp, 16u * b0);
@@ -578,7 +583,6 @@ __device__ __forceinline__ void g8_tile(const PfGemm& a, const PfSeg& sg, int n0
 
     // D lane l: column l & 15, rows 4 (l >> 4) + e. The residual values are loaded together, from
     // clamped addresses, before the first store.
-    const float wun = F16 ? ldexpf(1.0f, -fe) : SC == G8_SC_STEP ? ldexpf(1.0f, sg.wexp) : MIN ? ldexpf(1.0f, sg.wexp + 6) : 1.0f;
     const bool add = a.add && blockIdx.z == 0;
     float* out = blockIdx.z == 0 ? sg.y
                                  : a.part + (size_t)(blockIdx.z - 1) * a.T * sg.ldy + (size_t)(sg.y - a.seg[0].y);
@@ -601,7 +605,7 @@ __device__ __forceinline__ void g8_tile(const PfGemm& a, const PfSeg& sg, int n0
 #pragma unroll
             for (int e = 0; e < 4; e++) {
                 const int t = tb + e;
-                const float r = (F16 ? blk : acc)[i][j][e] * (sxs[t - t0] * wun);  // undoes the scales: exact
+                const float r = (F16 ? blk : acc)[i][j][e] * sxs[t - t0];  // exact
                 if (t < a.T && n < sg.N) out[(size_t)t * sg.ldy + n] = add ? old[j][e] + r : r;
             }
         }
