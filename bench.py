@@ -6,7 +6,8 @@ seed, a 512-token random prompt prefilled in one batched pass (fllm_prefill), th
 at batch 1.
 A "step" is one decode token: the forward pass and the greedy argmax. The timed steps run as a
 device-side loop (each step's argmax is the next step's input token on the device, one graph
-launch per step, the tokens are read back after the last step); the same tokens come out of the
+launch per four steps once sixteen have run, per step before; the tokens are read back after the last step);
+the same tokens come out of the
 host loop (forward + argmax + 4-byte read-back per token), whose rate is reported beside it.
 
 Prints one JSON line with the decode throughput, a roofline entry for the dominant kernel and a
@@ -391,7 +392,7 @@ def profiler_roofline(args, bytes_per_launch, dom_name, steps_launches):
 
 FP32_MFMA_PEAK_TFLOPS = 157.3  # MI355X dense fp32 matrix peak
 FP16_MFMA_PEAK_TFLOPS = 2500.0  # MI355X dense fp16 matrix peak
-Q8_0_TYPE, Q4_K_TYPE, Q5_K_TYPE = 8, 12, 13
+F16_TYPE, Q4_0_TYPE, Q8_0_TYPE, Q4_K_TYPE, Q5_K_TYPE = 1, 2, 8, 12, 13
 
 
 def prefill_report(cfg, n, seconds, stages=None):
@@ -399,10 +400,11 @@ def prefill_report(cfg, n, seconds, stages=None):
     element-wise steps and the last token's LM head included, so every fraction is a lower bound).
     `tflops`: the reference's own arithmetic, 2 flop per weight per token plus the causal attention's
     4 * heads * head_dim flop per (query, key) pair. The projections run on the fp16 matrix cores:
-    a Q4_K or Q5_K matrix takes two fp16 products per weight (exact integer weights against the
-    activations' hi and lo halves) plus one min-term product per 256-element block (1/8 of a
-    product), a Q8_0 one two (its int8 codes against the hi and lo halves), any other three (Q6_K:
-    exact integer hi / lo weights; other types: hi / lo splits of both operands); `gemm` is those
+    of matrices of whole 256-element blocks per row a Q4_K or Q5_K one takes two fp16 products per
+    weight (exact integer weights against the activations' hi and lo halves) plus one min-term
+    product per block (1/8 of a product), a Q8_0, Q4_0 or F16 one two (codes or weights against the
+    hi and lo halves), any other three (Q6_K: exact integer hi / lo weights; other types, and rows
+    that are no whole blocks: hi / lo splits of both operands); `gemm` is those
     fp16 products' rate against the fp16 peak. Attention runs on the f32 matrix cores, one product
     per flop, except at head_dim 128 and 256, where it takes three fp16 products per flop (hi / lo
     splits of both operands, the lo lo product dropped) against the fp16 peak."""
@@ -422,12 +424,16 @@ def prefill_report(cfg, n, seconds, stages=None):
         pairs_w, n_win = pairs, 0
     attn = 4.0 * cfg["n_heads"] * hd * (pairs * (L - n_win) + pairs_w * n_win)
     flops = 2.0 * n * weights + attn
-    launches = [((qdim * H, ty["q"]), (kvdim * H, ty["k"]), (kvdim * H, ty["v"])), ((H * qdim, ty["o"]),),
-                ((F * H, ty["gate"]), (F * H, ty["up"])), ((H * F, ty["down"]),)]
-    def products(t):
-        return 2.125 if t in (Q4_K_TYPE, Q5_K_TYPE) else 2.0 if t == Q8_0_TYPE else 3.0
+    # (weights, type, columns) of each launch's matrices
+    launches = [((qdim * H, ty["q"], H), (kvdim * H, ty["k"], H), (kvdim * H, ty["v"], H)), ((H * qdim, ty["o"], qdim),),
+                ((F * H, ty["gate"], H), (F * H, ty["up"], H)), ((H * F, ty["down"], F),)]
 
-    fp16 = sum(products(t) * w for g in launches for w, t in g)
+    def products(t, cols):
+        if cols % 256:
+            return 3.0
+        return 2.125 if t in (Q4_K_TYPE, Q5_K_TYPE) else 2.0 if t in (Q8_0_TYPE, Q4_0_TYPE, F16_TYPE) else 3.0
+
+    fp16 = sum(products(t, c) * w for g in launches for w, t, c in g)
     fp16_tf = 2.0 * n * L * fp16 / seconds / 1e12
     tf = flops / seconds / 1e12
     out = {"tokens": n, "tok_s": round(n / seconds, 2), "tflops": round(tf, 2),
@@ -441,9 +447,9 @@ def prefill_report(cfg, n, seconds, stages=None):
             row = {"launches": st["launches"], "ms": round(st["ms"], 3)}
             if name in gemm_of:
                 g = gemm_of[name]
-                issued = sum(products(t) * w for w, t in g)
+                issued = sum(products(t, c) * w for w, t, c in g)
                 mf = 2.0 * n * L * issued / (st["ms"] * 1e-3) / 1e12
-                row.update(dtype="fp16", products=round(issued / sum(w for w, _ in g), 3), mfma_tflops=round(mf, 1),
+                row.update(dtype="fp16", products=round(issued / sum(w for w, _, _ in g), 3), mfma_tflops=round(mf, 1),
                            mfma_frac=round(mf / FP16_MFMA_PEAK_TFLOPS, 4))
             elif name == "pf_attention" and hd in (128, 256):
                 mf = 3.0 * attn / (st["ms"] * 1e-3) / 1e12
