@@ -46,7 +46,8 @@ struct PfGemm {
 };
 // With pending non-null, a K-split launch leaves its parts z > 0 in a.part and sets *pending to their
 // number (0 when unsplit) instead of adding them: the next kernel that reads y adds them first, in
-// order (launch_pf_split_norm, launch_pf_qkv_post, launch_pf_postnorm_add), or launch_pf_split_add does.
+// order (launch_pf_split_norm, launch_pf_split_act, launch_pf_qkv_post, launch_pf_postnorm_add), or
+// launch_pf_split_add does.
 hipError_t launch_pf_gemm(PfGemm a, int n_cu, hipStream_t st, int* pending = nullptr);
 // y[i] += part[0][i] + ... + part[nsp - 1][i] (in that order), slices of n floats
 hipError_t launch_pf_split_add(float* y, const float* part, int nsp, int64_t n, hipStream_t st);
@@ -54,7 +55,7 @@ hipError_t launch_pf_split_add(float* y, const float* part, int nsp, int64_t n, 
 // largest magnitude lies in [2^14, 2^15), and written as hi = fp16(x 2^e_t) (plane 0) and
 // lo = fp16(x 2^e_t - hi) (plane 1, at xh + T * ldh), 22 significant bits together; xs[t] = 2^-e_t.
 // After the two planes: the hi and lo halves of each 32-element group's sum of the scaled values
-// (xh + 2 T ldh: T rows of K / 32, then the lo plane), for the Q4_K form's min term. xh holds
+// (xh + 2 T ldh: T rows of K / 32, then the lo plane), for the Q4_K / Q5_K forms' min term. xh holds
 // 2 T (ldh + K / 32) halves.
 hipError_t launch_pf_split(const float* x, int ldx, int T, int K, _Float16* xh, int ldh, float* xs, hipStream_t st);
 // launch_pf_split of a row computed on the way, never written: RmsNorm / GemmaRmsNorm (kind 1) of
